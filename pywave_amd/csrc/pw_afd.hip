@@ -908,38 +908,6 @@ __global__ __launch_bounds__(64 * WAVES) void k_afd2d(Geo g, Step a)
         a.snap[(size_t)(x - g.nb) * g.nz1 + (z - g.nb)] = c;
 }
 
-// ---------------------------------------------------------------- pseudo-spectral step
-// psm2d/psm's update (pywave/src/wave_psp.c:518-581, :193-256) with the spectral Laplacian 'wave'
-// computed beforehand over the whole padded grid: the same leapfrog, injection, damping of both
-// levels, receivers and snapshots as the finite-difference step, on every cell of the updated
-// domain.  One thread per cell; D3 selects the y faces.
-template <bool D3>
-__global__ __launch_bounds__(256) void k_ps_update(Geo g, Step a, const float* __restrict__ wave)
-{
-    const int z = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int x = blockIdx.y * 4 + (threadIdx.x >> 6);
-    const int y = blockIdx.z;
-    if (z >= g.nz || x >= g.nx) return;
-    const long long j = (long long)y * g.ldxy + (long long)x * g.ldz + z;
-    const float u = a.cur[j];
-    const float vc = a.vv[j];
-    const float2 fzz = a.fz[z], fxx = a.fx[x];
-    const float2 fyy = D3 ? a.fy[y] : make_float2(1.f, 1.f);
-    const float p = D3 ? damp3(a.pv[j], fzz, fxx, fyy) : damp2(a.pv[j], fzz, fxx);
-    float c = u + (u - p);
-    c = c + wave[j] * vc;
-    c = inject(c, vc, a, z, x, y);
-    const int nby = D3 ? g.nb : 0;
-    const bool onrec = z == g.nb && x >= g.nb && x < g.nb + g.nx1 && y >= nby && y < nby + g.ny1;
-    const long long r = (long long)(y - nby) * g.nx1 + (x - g.nb);
-    if (a.tri && onrec) c = c + vc * a.tri[r];
-    c = D3 ? damp3(c, fzz, fxx, fyy) : damp2(c, fzz, fxx);
-    a.pv[j] = c;
-    if (a.rec && onrec) a.rec[r] = c;
-    if (a.snap && z >= g.nb && z < g.nb + g.nz1 && x >= g.nb && x < g.nb + g.nx1 && y >= nby && y < nby + g.ny1)
-        a.snap[((long long)(y - nby) * g.nx1 + (x - g.nb)) * g.nz1 + (z - g.nb)] = c;
-}
-
 // ---------------------------------------------------------------- helpers
 // vv = ((v*v)*dt)*dt on the padded layout from the clamp-expanded model velocity
 // (vel_expand, pywave/src/wave_abc.c:14-125, replicates the model edges into the boundary)
@@ -1374,8 +1342,7 @@ struct pw_afd {
     size_t field_elems = 0;
     long long resident[kNumVariants3] = {};  // co-resident blocks per 3D variant (0: not queried)
     float dz = 0.f, dx = 0.f, dy = 0.f;
-    PsLap* ps = nullptr;      // pseudo-spectral Laplacian (aps2d/aps3d) instead of the stencil
-    float* d_wave = nullptr;  // its output, field layout
+    PsLap* ps = nullptr;  // pseudo-spectral Laplacian (aps2d/aps3d) instead of the stencil
 };
 
 namespace {
@@ -1557,7 +1524,6 @@ void afd_free(pw_afd* p)
     if (p->d_fx) hipFree(p->d_fx);
     if (p->d_fy) hipFree(p->d_fy);
     if (p->d_src) hipFree(p->d_src);
-    if (p->d_wave) hipFree(p->d_wave);
     ps_destroy(p->ps);
 }
 
@@ -1873,16 +1839,11 @@ static int afd_enqueue(pw_afd* p, int tri, hipEvent_t* evs, int nsteps = 0, bool
             a.snap = snap_of(it);
             int rc = PW_OK;
             if (p->ps) {
-                // spectral Laplacian of C_n, then the update (the pair of launches is one step)
-                PW_HIP(ctx, ps_apply(p->ps, A, p->d_wave, s));
-                dim3 grid(pw::ceil_div(g.nz, 64), pw::ceil_div(g.nx, 4), g.ny);
-                if (p->ndim == 3)
-                    hipExtLaunchKernelGGL(k_ps_update<true>, grid, dim3(256), 0, s, evs ? evs[2 * k] : nullptr,
-                                          evs ? evs[2 * k + 1] : nullptr, 0, g, a, (const float*)p->d_wave);
-                else
-                    hipExtLaunchKernelGGL(k_ps_update<false>, grid, dim3(256), 0, s, evs ? evs[2 * k] : nullptr,
-                                          evs ? evs[2 * k + 1] : nullptr, 0, g, a, (const float*)p->d_wave);
-                PW_HIP(ctx, hipGetLastError());
+                const PsStep b{A, B, p->d_vv, p->d_fz, p->d_fx, p->d_fy, p->d_src, p->d_wav, a.tri, a.rec, a.snap,
+                               a.ns, a.nt, it, g.nz, g.nx, g.ny, g.nb, g.nz1, g.nx1, g.ny1};
+                if (done == 0) PW_HIP(ctx, ps_begin(p->ps, b, s));
+                PW_HIP(ctx, ps_step(p->ps, b, done + 1 == total, s, evs ? evs[2 * k] : nullptr,
+                                    evs ? evs[2 * k + 1] : nullptr));
             } else {
                 const int saved = p->variant;
                 if (two) p->variant = kLeanDefault;  // odd remainder: one single step
@@ -2076,10 +2037,6 @@ int pw_afd_set_spectral(pw_afd* p, int on)
     std::string err;
     p->ps = ps_create(g.nz2, g.nx2, g.ny2, g.ldz, g.ldxy, p->dz, p->dx, p->dy, err);
     if (!p->ps) PW_FAIL(ctx, PW_ERR_ARG, "set_spectral: " + err);
-    if (!p->d_wave) {
-        PW_HIP(ctx, hipMalloc(&p->d_wave, p->field_elems * 4));
-        PW_HIP(ctx, hipMemsetAsync(p->d_wave, 0, p->field_elems * 4, ctx->s()));
-    }
     return PW_OK;
 }
 

@@ -78,10 +78,27 @@ int check_finite(pw_ctx* ctx, const void* d, size_t n, int elem_bytes, const cha
 
 }  // namespace pw
 
-// Pseudo-spectral Laplacian of padded fields (pw_psp.hip): n1 (z, even, real transform), n2 (x),
+// Pseudo-spectral engine of padded fields (pw_psp.hip): n1 (z, even, real transform), n2 (x),
 // n3 (y; 1 in 2D) are the padded extents; fields use the plans' layout (z stride ldz, plane
-// stride ldxy).  ps_apply enqueues wave = IFFT(-(2 pi |k|)^2 FFT(field)) on stream s.
+// stride ldxy).  One time step on stream s: ps_begin puts the spectrum of a step's current field
+// in the engine's buffer (once per run); ps_step turns it into the spectral Laplacian
+// IFFT(-(2 pi |k|)^2 FFT(cur)), updates the field as psm2d/psm do and, unless the step is the
+// run's last, leaves the new field's spectrum for the next call.
 struct PsLap;
+struct PsStep {
+    const float* cur;               // C_n (damped)
+    float* pv;                      // in: C_{n-1}; out: C_{n+1}
+    const float* vv;                // v^2 dt^2, same layout
+    const float2 *fz, *fx, *fy;     // damping (lo, hi) per index
+    const int* src;                 // 3*ns: gz, gx, gy in padded coordinates
+    const float* wav;               // ns*nt
+    const float* tri;               // this step's receiver plane [ny1][nx1] or null
+    float* rec;                     // this step's receiver plane or null
+    float* snap;                    // this snapshot [ny1][nx1][nz1] or null
+    int ns, nt, it;
+    int nz, nx, ny, nb, nz1, nx1, ny1;  // updated domain, boundary width, model
+};
 PsLap* ps_create(int n1, int n2, int n3, int ldz, long long ldxy, float dz, float dx, float dy, std::string& err);
-hipError_t ps_apply(PsLap* P, const float* field, float* wave, hipStream_t s);
+hipError_t ps_begin(PsLap* P, const PsStep& a, hipStream_t s);
+hipError_t ps_step(PsLap* P, const PsStep& a, bool last, hipStream_t s, hipEvent_t e0, hipEvent_t e1);
 void ps_destroy(PsLap* P);

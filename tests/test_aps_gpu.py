@@ -100,3 +100,25 @@ def test_aps3d_other_factorisation_vs_oracle():
     p.run()
     out = p.output()
     assert np.array_equal(out.reshape(nt, nx, ny, order="F"), d.transpose(2, 1, 0))
+
+
+@pytest.mark.parametrize("shape", [(84, 83, 85), (147, 79, 90), (19, 115, 118), (3, 118, 115), (250, 3, 2)])
+def test_aps3d_lines_per_block_vs_oracle(shape):
+    # grids on which the z, x and y kernels run 16, 8, 4 and 1 lines per block (two levels a pass or
+    # one), with partial last blocks and radix-5 lengths (125) on x or y; same operations in the same
+    # order as the oracle, so equal
+    rng = np.random.default_rng(sum(shape))
+    nz, nx, ny = shape
+    vel = (1700 + 900 * rng.random(shape)).astype(np.float32)
+    nt, dt, nbt = 9, 0.001, 5
+    wav = rng.standard_normal((1, nt)).astype(np.float32)
+    s = [nx // 2, ny // 2, min(1, nz - 1)]
+    d, snaps, _ = O.afd3d(vel, nt, dt, 10.0, 11.0, 12.0, nbt, 0.03, s[:1], s[1:2], s[2:], wav, jsnap=8, ps=True)
+    p = AfdPlan(vel, (12.0, 10.0, 11.0), nt, dt, nbt, 0.03, 8, spectral=True)
+    p.set_sources(np.array(s + [25, 0.002, 1.0], np.float32), 1, wavelet=wav)
+    p.run()
+    out = p.output()
+    n = nt * nx * ny
+    assert np.array_equal(out[:n].reshape(nt, nx, ny, order="F"), d.transpose(2, 1, 0))
+    w = out[n:].reshape(nz, nx, ny, -1, order="F")
+    assert all(np.array_equal(w[..., k], snaps[k].transpose(2, 1, 0)) for k in range(w.shape[-1]))
