@@ -25,6 +25,7 @@
 #include <hip/hip_ext.h>
 
 #include "pw_internal.h"
+#include "pw_afd2d.h"
 
 namespace {
 
@@ -874,6 +875,13 @@ __global__ __launch_bounds__(64 * WAVES) void k_afd3d_2step(Geo g, Step2 a, int 
     }
 }
 
+// ---------------------------------------------------------------- 2D: K steps per launch
+template <int K, int S, int W>
+__global__ __launch_bounds__(64 * W) void k_afd2d_multi(pw2d::Steps a)
+{
+    pw2d::advance<K, S, W>(a, blockIdx.x, blockIdx.y);
+}
+
 // ---------------------------------------------------------------- 2D: one cell per lane
 template <int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void k_afd2d(Geo g, Step a)
@@ -1406,75 +1414,119 @@ int afd_launch_step(pw_afd* p, const Step& a, hipEvent_t e0 = nullptr, hipEvent_
     pw_ctx* ctx = p->ctx;
     hipStream_t s = ctx->s();
     const Geo& g = p->g;
-    if (p->ndim == 2) {
-        constexpr int W = 4;
-        dim3 grid(pw::ceil_div(g.nz, 64), pw::ceil_div(g.nx, W));
-        hipExtLaunchKernelGGL(k_afd2d<W>, grid, dim3(64 * W), 0, s, e0, e1, 0, g, a);
-    } else {
-        const int vi = p->variant >= 0 ? p->variant : default_variant(p);
-        const Variant3 v = kVariants3[vi];
-        if (!variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "3D kernel variant not applicable to this grid");
-        const int ntz = pw::ceil_div(g.nz, 64), ntx = pw::ceil_div(g.nx, v.tx);
-        int nyc = p->ny_chunk;
-        if (nyc <= 0) {
-            // as many y chunks per tile column as fit one round of co-resident blocks: every
-            // block starts at once (no tail round) and neighbours stream in step through L2
-            const long long tiles = (long long)ntz * ntx;
-            const long long cap = resident_blocks(p, vi);
-            const int nch = (int)std::max(1LL, cap / tiles);
-            nyc = std::max(8, pw::ceil_div(g.ny, nch));
-        }
-        if (v.lean >= 2 && v.lean <= 4) nyc = std::min(nyc, max_chunk_planes(g));  // chunk window < 2 GiB
-        const int nch = pw::ceil_div(g.ny, nyc);
-        const int nblk = ntz * ntx * nch;
-        const int grid = pw::ceil_div(nblk, 8) * 8;
-        switch (vi) {
+    const int vi = p->variant >= 0 ? p->variant : default_variant(p);
+    const Variant3 v = kVariants3[vi];
+    if (!variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "3D kernel variant not applicable to this grid");
+    const int ntz = pw::ceil_div(g.nz, 64), ntx = pw::ceil_div(g.nx, v.tx);
+    int nyc = p->ny_chunk;
+    if (nyc <= 0) {
+        // as many y chunks per tile column as fit one round of co-resident blocks: every
+        // block starts at once (no tail round) and neighbours stream in step through L2
+        const long long tiles = (long long)ntz * ntx;
+        const long long cap = resident_blocks(p, vi);
+        const int nch = (int)std::max(1LL, cap / tiles);
+        nyc = std::max(8, pw::ceil_div(g.ny, nch));
+    }
+    if (v.lean >= 2 && v.lean <= 4) nyc = std::min(nyc, max_chunk_planes(g));  // chunk window < 2 GiB
+    const int nch = pw::ceil_div(g.ny, nyc);
+    const int nblk = ntz * ntx * nch;
+    const int grid = pw::ceil_div(nblk, 8) * 8;
+    switch (vi) {
 #define PW_V3(I, TX_, W_)                                                                          \
     case I:                                                                                        \
-        hipExtLaunchKernelGGL((k_afd3d<TX_, W_>), dim3(grid), dim3(64 * W_), 0, s, e0, e1, 0, g, a, ntz, ntx, \
-                              nyc, nblk);                                                                  \
-        break;
-            PW_V3(0, 16, 4)
-            PW_V3(1, 8, 4)
-            PW_V3(2, 16, 8)
-            PW_V3(3, 32, 8)
-            PW_V3(4, 8, 8)
-            PW_V3(5, 4, 4)
+    hipExtLaunchKernelGGL((k_afd3d<TX_, W_>), dim3(grid), dim3(64 * W_), 0, s, e0, e1, 0, g, a, ntz, ntx, \
+                          nyc, nblk);                                                                  \
+    break;
+        PW_V3(0, 16, 4)
+        PW_V3(1, 8, 4)
+        PW_V3(2, 16, 8)
+        PW_V3(3, 32, 8)
+        PW_V3(4, 8, 8)
+        PW_V3(5, 4, 4)
 #undef PW_V3
 #define PW_VL(I, TX_, W_)                                                                          \
     case I:                                                                                        \
-        hipExtLaunchKernelGGL((k_afd3d_lean<TX_ / W_, W_>), dim3(grid), dim3(64 * W_), 0, s, e0, e1, 0, g, a, \
-                              ntz, ntx, nyc, nblk);                                                             \
-        break;
-            PW_VL(6, 16, 8)
-            PW_VL(7, 8, 8)
-            PW_VL(8, 16, 4)
-            PW_VL(9, 32, 8)
-            PW_VL(10, 16, 16)
-            PW_VL(11, 32, 16)
+    hipExtLaunchKernelGGL((k_afd3d_lean<TX_ / W_, W_>), dim3(grid), dim3(64 * W_), 0, s, e0, e1, 0, g, a, \
+                          ntz, ntx, nyc, nblk);                                                             \
+    break;
+        PW_VL(6, 16, 8)
+        PW_VL(7, 8, 8)
+        PW_VL(8, 16, 4)
+        PW_VL(9, 32, 8)
+        PW_VL(10, 16, 16)
+        PW_VL(11, 32, 16)
 #undef PW_VL
 #define PW_VP(I, TX_, W_, NT_, ORD_)                                                                \
     case I:                                                                                         \
-        hipExtLaunchKernelGGL((k_afd3d_pipe<TX_ / W_, W_, NT_, ORD_>), dim3(grid), dim3(64 * W_), 0, s, e0, e1, \
-                              0, g, a, ntz, ntx, nyc, nblk);                                                         \
-        break;
-            PW_VP(12, 16, 8, 0, 0)
-            PW_VP(13, 16, 4, 0, 0)
-            PW_VP(14, 32, 8, 0, 0)
-            PW_VP(15, 8, 4, 0, 0)
-            PW_VP(16, 16, 8, 1, 0)
-            PW_VP(17, 16, 4, 1, 0)
-            PW_VP(18, 32, 16, 0, 0)
-            PW_VP(19, 8, 8, 0, 0)
-            PW_VP(20, 16, 4, 0, 1)
-            PW_VP(21, 8, 4, 0, 1)
-            PW_VP(22, 16, 8, 0, 1)
-            PW_VP(23, 32, 8, 0, 1)
+    hipExtLaunchKernelGGL((k_afd3d_pipe<TX_ / W_, W_, NT_, ORD_>), dim3(grid), dim3(64 * W_), 0, s, e0, e1, \
+                          0, g, a, ntz, ntx, nyc, nblk);                                                         \
+    break;
+        PW_VP(12, 16, 8, 0, 0)
+        PW_VP(13, 16, 4, 0, 0)
+        PW_VP(14, 32, 8, 0, 0)
+        PW_VP(15, 8, 4, 0, 0)
+        PW_VP(16, 16, 8, 1, 0)
+        PW_VP(17, 16, 4, 1, 0)
+        PW_VP(18, 32, 16, 0, 0)
+        PW_VP(19, 8, 8, 0, 0)
+        PW_VP(20, 16, 4, 0, 1)
+        PW_VP(21, 8, 4, 0, 1)
+        PW_VP(22, 16, 8, 0, 1)
+        PW_VP(23, 32, 8, 0, 1)
 #undef PW_VP
-            default:
-                PW_FAIL(ctx, PW_ERR_ARG, "unknown 3D kernel variant");
-        }
+        default:
+            PW_FAIL(ctx, PW_ERR_ARG, "unknown 3D kernel variant");
     }
+    PW_HIP(ctx, hipGetLastError());
+    return PW_OK;
+}
+
+// 2D launch shapes: steps per launch K, columns per strip, strips per tile.  A tile recomputes its
+// growth of 2K cells a side, so on small grids, where every tile has a CU of its own, the launch's
+// fixed cost (about 3 us) is spread over K = 8 steps and the narrowest tiles that fit the chip at
+// once are the fastest; once tiles queue, the redundant cells count and K = 4 wins.  Measured, us
+// per step (one step per launch 2.9, 3.2, 3.5, 9.5 on the same grids):
+//   updated grid   161^2   263 x 457   480^2   1060 x 1560
+//   8, 4 x 10       1.24      1.79      2.66      14.1
+//   8, 4 x 12       1.27      1.36      1.67       7.3
+//   8, 4 x 16       1.45      1.51      1.55       7.3
+//   4, 4 x 8        1.75      1.78      1.92       5.2
+struct Shape2 {
+    int k, owned_z, owned_x;
+};
+constexpr Shape2 kShapes2[] = {{8, 32, 8}, {8, 32, 16}, {8, 32, 32}, {4, 48, 16}};
+constexpr int kTilesAtOnce = 280;  // 256 CUs, and a few tiles that share one
+
+int shape2_of(const Geo& g)
+{
+    for (int i = 0; i < 3; ++i)
+        if ((long long)pw::ceil_div(g.nz, kShapes2[i].owned_z) * pw::ceil_div(g.nx, kShapes2[i].owned_x) <= kTilesAtOnce)
+            return i;
+    return 3;
+}
+
+int afd_launch_multi(pw_afd* p, int shape, const pw2d::Steps& a, hipEvent_t e0, hipEvent_t e1)
+{
+    pw_ctx* ctx = p->ctx;
+    hipStream_t s = ctx->s();
+    const Geo& g = p->g;
+#define PW_M2(I, K, S, W)                                                                                      \
+    case I: {                                                                                                  \
+        using T = pw2d::Tile<K, S, W>;                                                                         \
+        static_assert(kShapes2[I].k == K && kShapes2[I].owned_z == T::owned_z &&                               \
+                      kShapes2[I].owned_x == T::owned_x, "launch shape");                                      \
+        const dim3 grid(pw::ceil_div(g.nz, T::owned_z), pw::ceil_div(g.nx, T::owned_x));                       \
+        hipExtLaunchKernelGGL((k_afd2d_multi<K, S, W>), grid, dim3(64 * W), 0, s, e0, e1, 0, a);               \
+        break;                                                                                                 \
+    }
+    switch (shape) {
+        PW_M2(0, 8, 4, 10)
+        PW_M2(1, 8, 4, 12)
+        PW_M2(2, 8, 4, 16)
+        PW_M2(3, 4, 4, 8)
+        default: PW_FAIL(ctx, PW_ERR_ARG, "unknown 2D launch shape");
+    }
+#undef PW_M2
     PW_HIP(ctx, hipGetLastError());
     return PW_OK;
 }
@@ -1630,9 +1682,12 @@ pw_afd* pw_afd_create(pw_ctx* ctx, int ndim, int nz, int nx, int ny, float dz, f
     p->chunk_ok = lean && max_chunk_planes(g) >= 1;
 
     const size_t nrec = (size_t)g.nx1 * g.ny1;
-    bool ok = hipMalloc(&p->raw[0], p->raw_elems * 4) == hipSuccess &&
-              hipMalloc(&p->raw[1], p->raw_elems * 4) == hipSuccess &&
-              hipMalloc(&p->raw[2], p->raw_elems * 4) == hipSuccess &&
+    // 3D: three fields (two more when a two-step kernel first runs); 2D: the five fields of the
+    // multi-step launches in one allocation, as its cost counts in a one-shot call on a small grid
+    const size_t nfield = ndim == 2 ? 5 : 1;
+    bool ok = hipMalloc(&p->raw[0], nfield * p->raw_elems * 4) == hipSuccess &&
+              (ndim == 2 || (hipMalloc(&p->raw[1], p->raw_elems * 4) == hipSuccess &&
+                             hipMalloc(&p->raw[2], p->raw_elems * 4) == hipSuccess)) &&
               hipMalloc(&p->d_fz, fz.size() * 4) == hipSuccess &&
               hipMalloc(&p->d_fx, fx.size() * 4) == hipSuccess &&
               hipMalloc(&p->d_fy, fy.size() * 4) == hipSuccess &&
@@ -1642,9 +1697,17 @@ pw_afd* pw_afd_create(pw_ctx* ctx, int ndim, int nz, int nx, int ny, float dz, f
         ok = hipMalloc(&p->d_fz1, fz1.size() * 4) == hipSuccess && hipMalloc(&p->d_fx1, fx1.size() * 4) == hipSuccess &&
              hipMalloc(&p->d_fy1, fy1.size() * 4) == hipSuccess;
     if (ok) {
-        p->d_a = p->raw[0] + p->guard_lo;
-        p->d_b = p->raw[1] + p->guard_lo;
-        p->d_vv = p->raw[2] + p->guard_lo;
+        if (ndim == 2) {
+            p->d_a = p->raw[0];
+            p->d_b = p->d_a + p->raw_elems;
+            p->d_vv = p->d_b + p->raw_elems;
+            p->d_c = p->d_vv + p->raw_elems;
+            p->d_d = p->d_c + p->raw_elems;
+        } else {
+            p->d_a = p->raw[0] + p->guard_lo;
+            p->d_b = p->raw[1] + p->guard_lo;
+            p->d_vv = p->raw[2] + p->guard_lo;
+        }
     }
     if (ok && p->ntsnap > 0)
         ok = hipMalloc(&p->d_snap, (size_t)p->ntsnap * g.nz1 * g.nx1 * g.ny1 * 4) == hipSuccess;
@@ -1658,7 +1721,7 @@ pw_afd* pw_afd_create(pw_ctx* ctx, int ndim, int nz, int nx, int ny, float dz, f
     ok = hipMemcpyAsync(p->d_fz, fz.data(), fz.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
          hipMemcpyAsync(p->d_fx, fx.data(), fx.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
          hipMemcpyAsync(p->d_fy, fy.data(), fy.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
-         hipMemsetAsync(p->raw[2], 0, p->raw_elems * 4, s) == hipSuccess &&
+         hipMemsetAsync(p->d_vv - p->guard_lo, 0, (ndim == 2 ? 3 : 1) * p->raw_elems * 4, s) == hipSuccess &&
          (!lean || (hipMemcpyAsync(p->d_fz1, fz1.data(), fz1.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
                     hipMemcpyAsync(p->d_fx1, fx1.data(), fx1.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
                     hipMemcpyAsync(p->d_fy1, fy1.data(), fy1.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess)) &&
@@ -1780,6 +1843,8 @@ static int afd_enqueue(pw_afd* p, int tri, hipEvent_t* evs, int nsteps = 0, bool
     hipStream_t s = ctx->s();
     const int vi = p->ndim == 3 && !p->ps ? (p->variant >= 0 ? p->variant : default_variant(p)) : -1;
     const bool two = vi >= 0 && kVariants3[vi].lean == 5;
+    const bool multi = p->ndim == 2 && !p->ps;
+    const int shape2 = multi ? shape2_of(g) : 0;
     if (two && !variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "two-step 3D kernel not applicable to this grid");
     if (two && !p->d_c) {
         PW_HIP(ctx, hipMalloc(&p->raw[3], p->raw_elems * 4));
@@ -1790,8 +1855,8 @@ static int afd_enqueue(pw_afd* p, int tri, hipEvent_t* evs, int nsteps = 0, bool
         p->d_d = p->raw[4] + p->guard_lo;
     }
     if (zero) {
-        PW_HIP(ctx, hipMemsetAsync(p->raw[0], 0, p->raw_elems * 4, s));
-        PW_HIP(ctx, hipMemsetAsync(p->raw[1], 0, p->raw_elems * 4, s));
+        PW_HIP(ctx, hipMemsetAsync(p->d_a - p->guard_lo, 0, p->raw_elems * 4, s));
+        PW_HIP(ctx, hipMemsetAsync(p->d_b - p->guard_lo, 0, p->raw_elems * 4, s));
     }
     const size_t nrec = (size_t)g.nx1 * g.ny1;
     const size_t snap_elems = (size_t)g.nz1 * g.nx1 * g.ny1;
@@ -1827,6 +1892,20 @@ static int afd_enqueue(pw_afd* p, int tri, hipEvent_t* evs, int nsteps = 0, bool
             A = Db; B = Cb; Cb = oa; Db = ob;
             it += 2 * its;
             done += 2;
+        } else if (multi) {
+            const int nk = std::min(kShapes2[shape2].k, total - done);
+            unsigned snaps = 0;
+            for (int j = 0; j < nk; ++j)
+                if (p->jsnap > 0 && (it + j * its) % p->jsnap == 0) snaps |= 1u << j;
+            const pw2d::Steps a{A, B, p->d_vv, Cb, Db, p->d_fz, p->d_fx, p->d_src, p->d_wav, tri ? p->d_tri : nullptr,
+                                tri ? nullptr : p->d_rec, p->d_snap, tri ? 0 : p->ns, p->nt, it,
+                                its, nk, p->jsnap, snaps, g.nz, g.nx, g.nz2, g.nx2, g.ldz, g.nb, g.nz1, g.nx1, g.idz, g.idx, g.cc};
+            int rc = afd_launch_multi(p, shape2, a, evs ? evs[2 * k] : nullptr, evs ? evs[2 * k + 1] : nullptr);
+            if (rc) return rc;
+            std::swap(A, Cb);
+            std::swap(B, Db);
+            it += nk * its;
+            done += nk;
         } else {
             Step a{};
             a.cur = A; a.pv = B; a.vv = p->d_vv;

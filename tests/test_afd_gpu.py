@@ -354,3 +354,32 @@ def test_errors_follow_reference():
     with pytest.raises(ValueError):  # stencil would leave the padded domain
         pywave_amd.afd2d(vel, nt=10, ax=[0, 10, 30], az=[0, 10, 20], ns=1, sx=[5], sz=[-1], f=[10],
                          t=[0.001], A=[1], nbt=0, jsnap=0)
+
+
+@pytest.mark.parametrize("tri", [False, True])
+@pytest.mark.parametrize("shape,nbt,nt", [((5, 7), 2, 3), ((100, 101), 30, 21), ((203, 397), 30, 13), ((380, 421), 31, 17),
+                                          ((640, 500), 7, 11), ((64, 33), 16, 9)])
+def test_afd2d_multi_step_launches_vs_oracle(shape, nbt, nt, tri):
+    # grids of every 2D launch shape (8- and 4-step launches of narrow to wide tiles), run lengths that
+    # leave a shorter last launch, sources at tile corners, snapshots at steps inside a launch; the
+    # same operations in the same order as the oracle's, so equal
+    rng = np.random.default_rng(sum(shape) + nt)
+    nz, nx = shape
+    vel = (1500 + 1500 * rng.random(shape)).astype(np.float32)
+    dt, dz, dx, jsnap = 0.001, 9.0, 11.0, 5
+    sx, sz = [nx // 2, min(nx - 1, 16)], [nz // 2, min(nz - 1, 32)]
+    wav = rng.standard_normal((2, nt)).astype(np.float32)
+    dat = rng.standard_normal((nt, nx)).astype(np.float32)
+    d, snaps, _ = O.afd2d(vel, nt, dt, dx, dz, nbt, 0.02, sx, sz, wav, tri=tri, dat=dat.T, jsnap=jsnap)
+    p = AfdPlan(vel, (dz, dx), nt, dt, nbt, 0.02, jsnap)
+    if tri:
+        p.set_tri_data(dat)
+    else:
+        p.set_sources(np.array(sx + sz + [20, 20, 0.002, 0.002, 1, 1], np.float32), 2, wavelet=wav)
+    for _ in range(2):  # a second run starts from zeroed fields
+        p.run(tri=tri)
+        out = p.output()
+        assert np.array_equal(out[:nt * nx].reshape(nt, nx, order="F"), dat if tri else d.T)
+        w = out[nt * nx:].reshape(nz, nx, -1, order="F")
+        assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
+    p.close()
