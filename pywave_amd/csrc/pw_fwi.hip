@@ -1910,6 +1910,7 @@ struct pw_fwi {
     int cur_b0 = 0;         // first shot of the batch set by set_batch
     std::string active_err; // why the point-source geometry is unusable (empty: usable)
     bool visco = false;     // visco-acoustic modelling and the gradient_v imaging gradient
+    bool modelling = false;  // models only: no data, adjoint, gradient or checkpoint storage (fwi_create)
     // tau, taus on the padded grid; forward memory variable R0/R1 and backward RB0/RB1 per slot;
     // the forward one at every checkpoint [segment][slot][fs]
     float *tau_pad = nullptr, *taus_pad = nullptr, *R0 = nullptr, *R1 = nullptr;
@@ -2350,7 +2351,7 @@ int tune_widths(pw_fwi* p)
         rc = pick([&](int W) { launch_fwd<T, false>(W, g, f, a.padnz, a.padnx, nb_, s); }, &p->w_fwd);
         // the exact gradient's forward steps also store their term (4 B more per cell, written
         // once): timed on their own, as the extra stream moves the best width
-        if (!rc) {
+        if (!rc && !p->modelling) {
             StepArgs<T> ft = f;
             ft.full = (T*)p->seg;
             ft.fulls = p->fs;
@@ -2381,6 +2382,10 @@ int tune_widths(pw_fwi* p)
             if (!wbest || ms < tbest) { tbest = ms; wbest = W; }
         }
         if (tbest < 2.f * t1 || p->force_fused) p->w_fwd2 = wbest;
+    }
+    if (p->modelling) {  // no adjoint runs
+        p->widths_tuned = true;
+        return PW_OK;
     }
     StepArgs<T> b = base_args<T>(p);
     b.X = (const T*)p->A; b.Y = (T*)p->B; b.it = a.nt - 1;
@@ -2450,7 +2455,7 @@ std::vector<long long> tune_key(const pw_fwi* p)
 {
     const Acq& a = p->acq;
     std::vector<long long> k = {2, (long long)p->prec, p->nslot, a.padnz, a.padnx, a.nt, a.nb, a.sz, a.rz,
-                                a.ns, a.acqui_type, a.ds_v, a.s0_v, a.dr_v, p->visco, p->passive,
+                                a.ns, a.acqui_type, a.ds_v, a.s0_v, a.dr_v, p->visco, p->passive, p->modelling,
                                 p->max_fused, p->force_fused, p->seg_cap >= 2LL * p->nslot * p->fs};
     k.insert(k.end(), a.r0_v.begin(), a.r0_v.end());
     k.insert(k.end(), a.nr2.begin(), a.nr2.end());
@@ -2910,10 +2915,27 @@ int dot_dev(pw_fwi* p, const void* x, const void* y, double* out)
 
 }  // namespace
 
+namespace {
+pw_fwi* fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precision, bool modelling);
+}
+
 // ==================================================================================== C ABI
 extern "C" {
 
 pw_fwi* pw_fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precision)
+{
+    return fwi_create(ctx, pararray, batch, precision, false);
+}
+
+}  // extern "C"
+
+namespace {
+
+// modelling: a plan that only ever models (the one-shot forward_modeling_ac and its visco-acoustic
+// counterpart) holds no data, adjoint or gradient buffers and no checkpoints: for 8 shots of
+// 400 x 800, 1000 steps, those are 15.5 GB, whose allocation on each call took 0 to 1.1 s of a
+// call that models for 20 ms.
+pw_fwi* fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precision, bool modelling)
 {
     if (!ctx || !pararray) return nullptr;
     if (precision != 4 && precision != 8) {
@@ -2927,6 +2949,7 @@ pw_fwi* pw_fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precisi
     pw_fwi* p = new pw_fwi;
     p->ctx = ctx;
     p->prec = precision;
+    p->modelling = modelling;
     std::string err;
     if (acq_from_pararray(pararray, p->acq, err)) {
         ctx->err = err;
@@ -2980,25 +3003,30 @@ pw_fwi* pw_fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precisi
     rc = rc ? rc : dmalloc(p, &p->wav, a.nt * e);
     rc = rc ? rc : dmalloc(p, &p->X, fld * e);
     rc = rc ? rc : dmalloc(p, &p->Y, fld * e);
-    rc = rc ? rc : dmalloc(p, &p->A, fld * e);
-    rc = rc ? rc : dmalloc(p, &p->B, fld * e);
+    rc = rc || modelling ? rc : dmalloc(p, &p->A, fld * e);
+    rc = rc || modelling ? rc : dmalloc(p, &p->B, fld * e);
     rc = rc ? rc : dmalloc(p, &p->rec, p->nslot * tr * e);
     rc = rc ? rc : dmalloc(p, &p->res, p->nslot * tr * e);
-    rc = rc ? rc : dmalloc(p, &p->obs, (size_t)a.ns * tr * e);
-    rc = rc ? rc : dmalloc(p, &p->W, tr * e);
-    rc = rc ? rc : dmalloc(p, &p->gm, fld * e);
-    rc = rc ? rc : dmalloc(p, &p->gslot, (size_t)p->nslot * p->nzx * e);
-    rc = rc ? rc : dmalloc(p, &p->gtot, p->nzx * 8);
-    rc = rc ? rc : dmalloc(p, (void**)&p->gfold, (size_t)a.nz * a.padnx * 8);
+    rc = rc || modelling ? rc : dmalloc(p, &p->obs, (size_t)a.ns * tr * e);
+    rc = rc || modelling ? rc : dmalloc(p, &p->W, tr * e);
+    rc = rc || modelling ? rc : dmalloc(p, &p->gm, fld * e);
+    rc = rc || modelling ? rc : dmalloc(p, &p->gslot, (size_t)p->nslot * p->nzx * e);
+    rc = rc || modelling ? rc : dmalloc(p, &p->gtot, p->nzx * 8);
+    rc = rc || modelling ? rc : dmalloc(p, (void**)&p->gfold, (size_t)a.nz * a.padnx * 8);
     rc = rc ? rc : dmalloc(p, &p->patch, (size_t)p->nslot * PMAX * PMAX * e);
-    rc = rc ? rc : dmalloc(p, (void**)&p->tmpv, p->nzx * 4);
-    rc = rc ? rc : dmalloc(p, (void**)&p->work, (size_t)std::max(a.nz, a.nx) * (std::max(a.nz, a.nx) + 8) * 4);
+    rc = rc ? rc : dmalloc(p, (void**)&p->tmpv, p->nzx * 4);  // upload_model writes it in every plan
+    rc = rc || modelling ? rc : dmalloc(p, (void**)&p->work, (size_t)std::max(a.nz, a.nx) * (std::max(a.nz, a.nx) + 8) * 4);
     rc = rc ? rc : dmalloc(p, (void**)&p->shots, sizeof(ShotInfo) * p->nslot);
     rc = rc ? rc : dmalloc(p, (void**)&p->slot_shot, sizeof(int) * p->nslot);
     rc = rc ? rc : dmalloc(p, (void**)&p->partial, 1024 * 8);
     rc = rc ? rc : dmalloc(p, (void**)&p->dscalar, 8);
     rc = rc ? rc : dmalloc(p, (void**)&p->dhash, 16);
-    if (!rc) rc = plan_storage(p, 0);
+    if (modelling) {
+        p->K = a.nt;
+        p->nseg = 1;
+    } else if (!rc) {
+        rc = plan_storage(p, 0);
+    }
     if (rc) {
         fwi_free(p);
         delete p;
@@ -3014,24 +3042,27 @@ pw_fwi* pw_fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precisi
         if (i < a.nb) sx[2 * i] = a.bc[i];
         if (i >= a.padnx - a.nb) sx[2 * i + 1] = a.bc[a.padnx - i - 1];
     }
-    std::vector<float> w;
-    residual_weights(a, w);
-    std::vector<float> wt((size_t)a.nt * a.nr);  // [it][ir]
-    for (int ir = 0; ir < a.nr; ++ir)
-        for (int it = 0; it < a.nt; ++it) wt[(size_t)it * a.nr + ir] = w[(size_t)ir * a.nt + it];
+    std::vector<float> wt;  // [it][ir]
+    if (!modelling) {
+        std::vector<float> w;
+        residual_weights(a, w);
+        wt.resize((size_t)a.nt * a.nr);
+        for (int ir = 0; ir < a.nr; ++ir)
+            for (int it = 0; it < a.nt; ++it) wt[(size_t)it * a.nr + ir] = w[(size_t)ir * a.nt + it];
+    }
     hipStream_t s = ctx->s();
     bool ok;
     if (precision == 4) {
         std::vector<float> fz(sz.begin(), sz.end()), fx(sx.begin(), sx.end());
         ok = hipMemcpyAsync(p->sfz, fz.data(), fz.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
              hipMemcpyAsync(p->sfx, fx.data(), fx.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
-             hipMemcpyAsync(p->W, wt.data(), wt.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
+             (modelling || hipMemcpyAsync(p->W, wt.data(), wt.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess) &&
              hipStreamSynchronize(s) == hipSuccess;
     } else {
         std::vector<double> wd(wt.begin(), wt.end());
         ok = hipMemcpyAsync(p->sfz, sz.data(), sz.size() * 8, hipMemcpyHostToDevice, s) == hipSuccess &&
              hipMemcpyAsync(p->sfx, sx.data(), sx.size() * 8, hipMemcpyHostToDevice, s) == hipSuccess &&
-             hipMemcpyAsync(p->W, wd.data(), wd.size() * 8, hipMemcpyHostToDevice, s) == hipSuccess &&
+             (modelling || hipMemcpyAsync(p->W, wd.data(), wd.size() * 8, hipMemcpyHostToDevice, s) == hipSuccess) &&
              hipStreamSynchronize(s) == hipSuccess;
     }
     if (!ok) {
@@ -3042,6 +3073,10 @@ pw_fwi* pw_fwi_create(pw_ctx* ctx, const float* pararray, int batch, int precisi
     }
     return p;
 }
+
+}  // namespace
+
+extern "C" {
 
 void pw_fwi_destroy(pw_fwi* p)
 {
@@ -3233,9 +3268,9 @@ int pw_fwi_set_visco(pw_fwi* p, const float* q)
     if (!rc && !p->taus_pad) rc = dmalloc(p, (void**)&p->taus_pad, p->fs * 4);
     if (!rc && !p->R0) rc = dmalloc(p, (void**)&p->R0, fld * 4);
     if (!rc && !p->R1) rc = dmalloc(p, (void**)&p->R1, fld * 4);
-    if (!rc && !p->RB0) rc = dmalloc(p, (void**)&p->RB0, fld * 4);
-    if (!rc && !p->RB1) rc = dmalloc(p, (void**)&p->RB1, fld * 4);
-    if (!rc && !p->ckpt_r) rc = dmalloc(p, (void**)&p->ckpt_r, (size_t)p->nseg * fld * 4);
+    if (!rc && !p->modelling && !p->RB0) rc = dmalloc(p, (void**)&p->RB0, fld * 4);
+    if (!rc && !p->modelling && !p->RB1) rc = dmalloc(p, (void**)&p->RB1, fld * 4);
+    if (!rc && !p->modelling && !p->ckpt_r) rc = dmalloc(p, (void**)&p->ckpt_r, (size_t)p->nseg * fld * 4);
     if (rc) return rc;
     hipStream_t s = p->ctx->s();
     PW_HIPS(hipMemcpyAsync(p->tau_pad, tap.data(), tap.size() * 4, hipMemcpyHostToDevice, s));
@@ -3731,7 +3766,7 @@ int pw_forward_modeling_ac(pw_ctx* ctx, const float* vel, const float* q, const 
     std::string err;
     if (acq_from_pararray(pararray, a, err)) PW_FAIL(ctx, PW_ERR_ARG, err);
     if (out_len != (long long)a.nt * a.nx * a.ns) PW_FAIL(ctx, PW_ERR_ARG, "forward_modeling_ac: output length");
-    pw_fwi* p = pw_fwi_create(ctx, pararray, 0, 4);
+    pw_fwi* p = fwi_create(ctx, pararray, 0, 4, true);
     if (!p) return PW_ERR_ARG;
     int rc = pw_fwi_set_wavelet(p, wav);
     if (!rc) rc = pw_fwi_forward(p, vel, out);
@@ -3750,7 +3785,7 @@ int pw_forward_modeling_c(pw_ctx* ctx, const float* vel, const float* q, const f
     std::string err;
     if (acq_from_pararray(pararray, a, err)) PW_FAIL(ctx, PW_ERR_ARG, err);
     if (out_len != (long long)a.nt * a.nx * a.ns) PW_FAIL(ctx, PW_ERR_ARG, "forward_modelingc: output length");
-    pw_fwi* p = pw_fwi_create(ctx, pararray, 0, 4);
+    pw_fwi* p = fwi_create(ctx, pararray, 0, 4, true);
     if (!p) return PW_ERR_ARG;
     int rc = pw_fwi_set_wavelet(p, wav);
     if (!rc) rc = pw_fwi_set_visco(p, q);
