@@ -1364,10 +1364,21 @@ int max_chunk_planes(const Geo& g)
 }
 
 // the 3D kernel used when none was chosen
+// Tiles of 8 rows, 4 waves a block, while the three fields stay in the Infinity Cache (many small
+// blocks keep more of a plane's latencies in flight), of 16 rows beyond it (fewer halo re-reads):
+// with default_chunk, us per step on 91^3, 141^3, 201^3, 261^3 and 321^3 updated cells 6.7, 12.8,
+// 25.3, 42.7 and 122 with 8 rows, 100 at 321^3 with 16; one round of resident blocks of 16 rows,
+// 8 waves, the former choice, 11.5, 15.5, 31.4, 52 and 141.
 int default_variant(const pw_afd* p)
 {
-    return p->chunk_ok ? kLeanDefault : (p->lean_ok ? kLeanOnlyDefault : kGeneralDefault);
+    if (p->chunk_ok) return 3.0 * 4.0 * (double)p->field_elems <= kCacheFitBytes ? 15 : 17;
+    return p->lean_ok ? kLeanOnlyDefault : kGeneralDefault;
 }
+
+// y planes per block with default_variant's pipelined kernels: about 35 chunks, of 3 to 8 planes.  The
+// best of 2 to 24 planes was 3, 3, 4, 5, 6, 6 and 8 on 91^3, 110^3, 141^3, 170^3, 201^3, 230^3 and
+// 261^3 updated cells, 5 on 141 x 100 x 160, 8 on 321^3.
+int default_chunk(const Geo& g) { return std::min(8, std::max(3, (g.ny + 17) / 35)); }
 
 // whether 3D variant vi can run on this plan's grid
 bool variant_ok(const pw_afd* p, int vi)
@@ -1419,6 +1430,7 @@ int afd_launch_step(pw_afd* p, const Step& a, hipEvent_t e0 = nullptr, hipEvent_
     if (!variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "3D kernel variant not applicable to this grid");
     const int ntz = pw::ceil_div(g.nz, 64), ntx = pw::ceil_div(g.nx, v.tx);
     int nyc = p->ny_chunk;
+    if (nyc <= 0 && p->variant < 0 && v.lean >= 2 && v.lean <= 4) nyc = default_chunk(g);
     if (nyc <= 0) {
         // as many y chunks per tile column as fit one round of co-resident blocks: every
         // block starts at once (no tail round) and neighbours stream in step through L2
