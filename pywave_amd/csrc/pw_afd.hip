@@ -2529,15 +2529,33 @@ int tri_tune(pw_tri* p)
     return PW_OK;
 }
 
+// The sweep's outcome depends on the grid and the groups per launch only; plans of one context
+// share it.  (tri3d_image makes a plan per call: 36 shapes of 8 launches, 24 ms, ran in front of
+// each 128^3 image.)
 int tri_ensure_tuned(pw_tri* p)
 {
     if (p->tuned || !p->pipe_ok) return PW_OK;
-    switch (std::min(kTriPassGroups, p->G)) {
-        case 1: return tri_tune<1>(p);
-        case 2: return tri_tune<2>(p);
-        case 3: return tri_tune<3>(p);
-        default: return tri_tune<4>(p);
+    const Geo& g = p->g;
+    const int gk = std::min(kTriPassGroups, p->G);
+    const std::vector<long long> key = {4, gk, g.nz, g.nx, g.ny};
+    auto hit = p->ctx->tuned2d.find(key);
+    if (hit != p->ctx->tuned2d.end()) {
+        p->tri_w = hit->second.first[0];
+        p->tri_nyc = hit->second.first[1];
+        p->tri_nt = hit->second.first[2];
+        p->tune_log = hit->second.second;
+        p->tuned = true;
+        return PW_OK;
     }
+    int rc;
+    switch (gk) {
+        case 1: rc = tri_tune<1>(p); break;
+        case 2: rc = tri_tune<2>(p); break;
+        case 3: rc = tri_tune<3>(p); break;
+        default: rc = tri_tune<4>(p); break;
+    }
+    if (!rc) p->ctx->tuned2d[key] = {{p->tri_w, p->tri_nyc, p->tri_nt}, p->tune_log};
+    return rc;
 }
 
 // one back-propagation of G groups, the pass-th group of passes (groups pass*kTriPassGroups ...)
