@@ -262,17 +262,17 @@ int pw_lstri_invert(pw_lstri *p, const float *data, int niter, float *src, int *
 int pw_lstri_use_graph(pw_lstri *p, int on);
 /* time steps per sweep launch: 1, 2, 4, or 0 for the plan's choice (timed before its first sweep
  * of each shot count: single-step tile widths 1-16, two-step launches and four-step launches of
- * 4- and 8-column tiles on the plan's own grid); identical results either way.  No counterpart in the reference (a scheduling choice of this
+ * 4 and 8 columns per wave on the plan's own grid); identical results either way.  No counterpart in the reference (a scheduling choice of this
  * engine). */
 int pw_lstri_steps_per_launch(pw_lstri *p, int n);
 /* single-step tile width (x columns per 64-cell tile): 1, 2, 4, 8, 16, or 0 for the plan's timed
  * choice; identical results either way.  No counterpart in the reference. */
 int pw_lstri_set_tile_width(pw_lstri *p, int w);
-/* output columns of the four-step launches' tiles: 4, 8, or 0 for the timed choice (identical
+/* columns per wave of the four-step launches: 4 (tiles of 16), 8 (of 32), or 0 for the timed choice (identical
  * results).  No counterpart in the reference. */
 int pw_lstri_set_four_step_columns(pw_lstri *p, int c);
 /* the last sweep's launch choice: w[0] single-step tile width, w[1] steps per launch, w[2] the
- * four-step tiles' output columns (3 ints); the timing sweep's (kernel, width, ms per launch)
+ * four-step launches' columns per wave (3 ints); the timing sweep's (kernel, width, ms per launch)
  * triples into log[3*cap] (kernel 0 modelling step, 1 adjoint step, 2 two-step modelling launch,
  * 3 two-step adjoint launch, 4 four-step modelling launch, 5 four-step adjoint launch); returns
  * their number.  No counterpart in the reference. */

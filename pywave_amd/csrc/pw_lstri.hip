@@ -456,16 +456,25 @@ __global__ __launch_bounds__(T2) void k_tr2(TriGeo g, TriArgs2 a, int ntz2)
 }
 
 // ---------------------------------------------------------------- NS time steps per launch
-// The two-step scheme carried to NS steps: a block owns an OZN x OX tile and stages the current
-// level on the tile grown by 4*NS cells.  Step k (1..NS) forms its level on the tile grown by
-// 4*(NS-k), reading the level before it through the stencil and the one before that pointwise, so
-// two LDS level buffers suffice: A holds the even levels (the staged current level, then 2, ...),
-// B the odd ones (the previous level as staged, then 1, 3, ...), and a step overwrites, cell by
-// cell, the level it reads pointwise.  Every cell uses the single-step kernels' expressions, so each
-// level equals NS single steps bit for bit.  The last two levels go to the spare fields C (step
-// NS-1) and D (step NS).
-constexpr int OZN = 56;  // output z per tile
-constexpr int TN = 1024;  // threads per block (16 waves: the LDS reads of the steps need them in flight)
+// A block advances the OZN x OX cells it owns NS steps.  It holds them grown by G = 4*NS cells on
+// every side: lanes run along z (64 = OZN + 2G), each of its waves owns a strip of S columns, and
+// both levels, v^2dt^2 and the decay factors of a cell stay in its thread's registers.  Once per
+// step every strip publishes the level the stencil reads (modelling: the level; adjoint: its
+// product with v^2dt^2) in LDS, reads its neighbours along z and across the strip edges, and
+// forms the new level with the single-step kernels' expressions, so each level equals single
+// steps bit for bit.  Cells of the growth whose values are no longer needed go stale; strips of
+// only such columns stop computing.  The source planes are loaded one step ahead.  The last two
+// levels go to the spare fields C (step NS-1) and D (step NS).
+//
+// Bound by the VALU work of one tile's steps and their LDS latency.  Measured on the 250 x 454
+// grid, four steps a launch: 8.4 us modelling and 8.2 us adjoint with 4-column strips, against
+// 13.4 and 11.0 us for a tile kept wholly in LDS (1024 threads over 88 x 40 cells of four arrays),
+// which read 16 neighbours of each cell and recomputed its indexes every step.
+constexpr int NSN = 4;                  // steps per launch
+constexpr int OZN = 64 - 8 * NSN;       // output z per tile
+// tiles of 4-column strips own 16 columns (12 waves), of 8-column strips 32 (8 waves)
+constexpr int trn_owned(int sn) { return 4 * sn; }
+constexpr int trn_waves(int sn) { return (trn_owned(sn) + 8 * NSN) / sn; }
 
 template <int NS>
 struct TriArgsN {
@@ -482,203 +491,138 @@ struct TriArgsN {
     long long rss;
 };
 
-// cells of the region of step k (the tile grown by 4*(NS-k))
-template <int NS, int OX>
-__host__ __device__ constexpr int trn_zr(int k) { return OZN + 8 * (NS - k); }
-template <int NS, int OX>
-__host__ __device__ constexpr int trn_xr(int k) { return OX + 8 * (NS - k); }
-template <int NS, int OX>
-__host__ __device__ constexpr int trn_sp_off(int k)  // offset of step k's source plane in the staged planes
+template <bool ADJ, int NS, int S>
+__global__ __launch_bounds__(64 * trn_waves(S)) void k_trn(TriGeo g, TriArgsN<NS> a, int ntz)
 {
-    return k <= 1 ? 0 : trn_sp_off<NS, OX>(k - 1) + trn_zr<NS, OX>(k - 1) * trn_xr<NS, OX>(k - 1);
-}
-
-template <bool ADJ, int NS, int OX>
-__global__ __launch_bounds__(TN) void k_trn(TriGeo g, TriArgsN<NS> a, int ntz)
-{
-    static_assert(NS >= 2, "at least two steps");
-    constexpr int G = 4 * NS;
-    constexpr int ZA = OZN + 2 * G, XA = OX + 2 * G;              // staged region R_0
-    constexpr int ZB = OZN + 2 * (G - 4), XB = OX + 2 * (G - 4);  // R_1
-    constexpr int NSP = ADJ ? 1 : trn_sp_off<NS, OX>(NS + 1);     // staged source planes
-    __shared__ float LA[XA][ZA + 1];                 // even levels, on R_0 coordinates
-    __shared__ float LB[XB][ZB + 1];                 // the staged previous level, then the odd levels (R_1)
-    __shared__ float PA[ADJ ? XA : 1][ZA + 1];       // adjoint: level x v^2dt^2
-    __shared__ float PB[ADJ ? XB : 1][ZB + 1];
-    __shared__ float VV[XA][ZA + 1];                 // v^2dt^2 on R_0
-    __shared__ float SP[NSP];                        // modelling: each step's source plane on its region
-    __shared__ float fz[ZA][2], fx[XA][2];           // decay factor pairs of R_0's rows and columns
-    __shared__ float rd[ADJ ? NS : 1][XB];           // adjoint: each step's injected row over R_1's columns
+    constexpr int G = 4 * NS, OX = trn_owned(S), NX = S * trn_waves(S);
+    static_assert(NX == OX + 2 * G && OZN == 64 - 2 * G && NS * S <= 64, "tile");
+    __shared__ float lds[2][NX * 64 + 8];  // four cells of guard at either end
     const int slot = blockIdx.y;
     const int tz = blockIdx.x % ntz, tx = blockIdx.x / ntz;
-    const int zo = tz * OZN, xo = tx * OX;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int z = tz * OZN - G + lane, c0 = w * S, xs = tx * OX - G + c0;
     const long long so = slot * g.fs;
-    const float* __restrict__ X = a.X + so;
-    const float* __restrict__ Y = a.Y + so;
-    auto ing = [&](int z, int x) { return z >= 0 && z < g.pz && x >= 0 && x < g.px; };
-    auto inr = [&](int z, int x) { return z >= 4 && z < g.pz - 4 && x >= 4 && x < g.px - 4; };
-    auto mz = [&](int z) { return z >= g.nb && z < g.nb + g.nz; };
-    auto mx = [&](int x) { return x >= g.nb && x < g.nb + g.nx; };
-    auto own = [&](int z, int x) { return z >= zo && z < zo + OZN && x >= xo && x < xo + OX; };
-    auto mi = [&](int z, int x) { return slot * a.pss + (long long)(x - g.nb) * g.nz + (z - g.nb); };
-    // ---- stage: current level, v^2dt^2 (and their product) on R_0, the previous level on R_1,
-    // the decay pairs, and each step's source plane (modelling) or injected row (adjoint).  Every
-    // global operand is loaded into registers first (all loads in flight together), then written
-    // to LDS, so the launch waits on memory once.
-    constexpr int N0 = (ZA * XA + TN - 1) / TN, N1 = (ZB * XB + TN - 1) / TN, NP = (NSP + TN - 1) / TN;
-    float r0[N0], rv[N0], r1[N1], rp[ADJ ? 1 : NP];
+    const bool zing = z >= 0 && z < g.pz, zinr = z >= 4 && z < g.pz - 4, zmod = z >= g.nb && z < g.nb + g.nz;
+    const bool zown = lane >= G && lane < 64 - G && zing;
+    float u[S], p[S], vc[S], fx[S], sv[S];
+    unsigned mask[S];  // cells the stencil updates (the 4-cell rim and cells off the grid stay zero)
+    const float fz = zing ? a.sfz[2 * z] * a.sfz[2 * z + 1] : 1.f;  // one of a pair is 1
+    const int zm = z - g.nb;
 #pragma unroll
-    for (int j = 0; j < N0; ++j) {
-        const int e = threadIdx.x + j * TN;
-        const int zz = e % ZA, xx = e / ZA;
-        const int z = zo - G + zz, x = xo - G + xx;
-        const bool in = e < ZA * XA && ing(z, x);
-        const long long k = (long long)x * g.ldz + z;
-        r0[j] = in ? X[k] : 0.f;
-        rv[j] = in ? a.v2[k] : 0.f;
-    }
-#pragma unroll
-    for (int j = 0; j < N1; ++j) {
-        const int e = threadIdx.x + j * TN;
-        const int zz = e % ZB, xx = e / ZB;
-        const int z = zo - G + 4 + zz, x = xo - G + 4 + xx;
-        r1[j] = (e < ZB * XB && ing(z, x)) ? Y[(long long)x * g.ldz + z] : 0.f;
-    }
-    if constexpr (!ADJ) {
-        // flat index over the steps' regions back to back: step k's region at trn_sp_off(k)
-#pragma unroll
-        for (int j = 0; j < NP; ++j) {
-            const int e = threadIdx.x + j * TN;
-            int k = 1;
-            while (k < NS && e >= trn_sp_off<NS, OX>(k + 1)) ++k;
-            const int zr = trn_zr<NS, OX>(k), el = e - trn_sp_off<NS, OX>(k);
-            const int zz = el % zr, xx = el / zr;
-            const int z = zo - 4 * (NS - k) + zz, x = xo - 4 * (NS - k) + xx;
-            rp[j] = (e < NSP && ing(z, x) && mz(z) && mx(x)) ? a.plane[k - 1][mi(z, x)] : 0.f;
-        }
-    } else {
-        for (int e = threadIdx.x; e < NS * XB; e += TN) {
-            const int k = e / XB, xx = e % XB;
-            const int x = xo - G + 4 + xx;
-            rd[k][xx] = (x >= 0 && x < g.px && mx(x)) ? a.row[k][slot * a.rss + (x - g.nb)] : 0.f;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < N0; ++j) {
-        const int e = threadIdx.x + j * TN;
-        if (e < ZA * XA) {
-            const int zz = e % ZA, xx = e / ZA;
-            LA[xx][zz] = r0[j];
-            VV[xx][zz] = rv[j];
-            if constexpr (ADJ) PA[xx][zz] = r0[j] * rv[j];
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < N1; ++j) {
-        const int e = threadIdx.x + j * TN;
-        if (e < ZB * XB) LB[e / ZB][e % ZB] = r1[j];
-    }
-    if constexpr (!ADJ) {
-#pragma unroll
-        for (int j = 0; j < NP; ++j) {
-            const int e = threadIdx.x + j * TN;
-            if (e < NSP) SP[e] = rp[j];
-        }
-    }
-    for (int t = threadIdx.x; t < ZA + XA; t += TN) {
-        if (t < ZA) {
-            const int z = zo - G + t;
-            const bool zv = z >= 0 && z < g.pz;
-            fz[t][0] = zv ? a.sfz[2 * z] : 1.f;
-            fz[t][1] = zv ? a.sfz[2 * z + 1] : 1.f;
-        } else {
-            const int u = t - ZA, x = xo - G + u;
-            const bool xv = x >= 0 && x < g.px;
-            fx[u][0] = xv ? a.sfx[2 * x] : 1.f;
-            fx[u][1] = xv ? a.sfx[2 * x + 1] : 1.f;
-        }
-    }
-    __syncthreads();
-    // ---- steps 1..NS
-#pragma unroll
-    for (int k = 1; k <= NS; ++k) {
-        const int zr = trn_zr<NS, OX>(k), xr = trn_xr<NS, OX>(k);
-        const int da = 4 * k, db = 4 * (k - 1);  // R_k's offsets in R_0 and R_1 coordinates
-        const bool odd = k & 1;                  // level k goes to B (odd) or A (even)
-        for (int e = threadIdx.x; e < zr * xr; e += TN) {
-            const int zz = e % zr, xx = e / zr;
-            const int z = zo - 4 * (NS - k) + zz, x = xo - 4 * (NS - k) + xx;
-            const int za = zz + da, xa = xx + da, zb = zz + db, xb = xx + db;
-            float v = 0.f, pv = 0.f;
-            if (ing(z, x)) {
-                const float zl = fz[za][0], zh = fz[za][1], xl = fx[xa][0], xh = fx[xa][1];
-                const float vv = VV[xa][za];
-                // the level before this step (stencil) and the one before that (pointwise)
-                const float u1 = odd ? LA[xa][za] : LB[xb][zb];
-                const float prev = odd ? LB[xb][zb] : LA[xa][za];
-                float u2 = 0.f;  // the 4-cell rim stays zero
-                if constexpr (!ADJ) {
-                    if (g.depth == z && mx(x) && own(z, x))  // record the level before the step
-                        a.row[k - 1][slot * a.rss + (x - g.nb)] = 0.f + u1;
-                    if (inr(z, x)) {
-                        float lx, lz;
-                        if (odd) {
-                            lx = W4 * (LA[xa + 4][za] + LA[xa - 4][za]) + W3 * (LA[xa + 3][za] + LA[xa - 3][za]) +
-                                 W2 * (LA[xa + 2][za] + LA[xa - 2][za]) + W1 * (LA[xa + 1][za] + LA[xa - 1][za]) +
-                                 W0 * u1;
-                            lz = W4 * (LA[xa][za + 4] + LA[xa][za - 4]) + W3 * (LA[xa][za + 3] + LA[xa][za - 3]) +
-                                 W2 * (LA[xa][za + 2] + LA[xa][za - 2]) + W1 * (LA[xa][za + 1] + LA[xa][za - 1]) +
-                                 W0 * u1;
-                        } else {
-                            lx = W4 * (LB[xb + 4][zb] + LB[xb - 4][zb]) + W3 * (LB[xb + 3][zb] + LB[xb - 3][zb]) +
-                                 W2 * (LB[xb + 2][zb] + LB[xb - 2][zb]) + W1 * (LB[xb + 1][zb] + LB[xb - 1][zb]) +
-                                 W0 * u1;
-                            lz = W4 * (LB[xb][zb + 4] + LB[xb][zb - 4]) + W3 * (LB[xb][zb + 3] + LB[xb][zb - 3]) +
-                                 W2 * (LB[xb][zb + 2] + LB[xb][zb - 2]) + W1 * (LB[xb][zb + 1] + LB[xb][zb - 1]) +
-                                 W0 * u1;
-                        }
-                        u2 = (lx * g.sx + lz * g.sz) * vv + 2.0f * u1 - decay(prev, zl, zh, xl, xh);
-                    }
-                    if (mz(z) && mx(x)) u2 = u2 + SP[trn_sp_off<NS, OX>(k) + e] * vv;
-                } else {
-                    const float c = odd ? PA[xa][za] : PB[xb][zb];  // the level before, x v^2dt^2
-                    if (mz(z) && mx(x) && own(z, x)) a.plane[k - 1][mi(z, x)] = 0.f + c;  // this step's image
-                    if (inr(z, x)) {
-                        float lx, lz;
-                        if (odd) {
-                            lx = W4 * (PA[xa + 4][za] + PA[xa - 4][za]) + W3 * (PA[xa + 3][za] + PA[xa - 3][za]) +
-                                 W2 * (PA[xa + 2][za] + PA[xa - 2][za]) + W1 * (PA[xa + 1][za] + PA[xa - 1][za]) +
-                                 W0 * c;
-                            lz = W4 * (PA[xa][za + 4] + PA[xa][za - 4]) + W3 * (PA[xa][za + 3] + PA[xa][za - 3]) +
-                                 W2 * (PA[xa][za + 2] + PA[xa][za - 2]) + W1 * (PA[xa][za + 1] + PA[xa][za - 1]) +
-                                 W0 * c;
-                        } else {
-                            lx = W4 * (PB[xb + 4][zb] + PB[xb - 4][zb]) + W3 * (PB[xb + 3][zb] + PB[xb - 3][zb]) +
-                                 W2 * (PB[xb + 2][zb] + PB[xb - 2][zb]) + W1 * (PB[xb + 1][zb] + PB[xb - 1][zb]) +
-                                 W0 * c;
-                            lz = W4 * (PB[xb][zb + 4] + PB[xb][zb - 4]) + W3 * (PB[xb][zb + 3] + PB[xb][zb - 3]) +
-                                 W2 * (PB[xb][zb + 2] + PB[xb][zb - 2]) + W1 * (PB[xb][zb + 1] + PB[xb][zb - 1]) +
-                                 W0 * c;
-                        }
-                        u2 = (lx * g.sx + lz * g.sz) + 2.0f * u1 - decay(prev, zl, zh, xl, xh);
-                    }
-                    if (z == g.depth && mx(x)) u2 = u2 + rd[k - 1][xb];
-                }
-                v = decay(u2, zl, zh, xl, xh);
-                if constexpr (ADJ) pv = v * vv;
-                if (k >= NS - 1 && own(z, x)) (k == NS ? a.D : a.C)[so + (long long)x * g.ldz + z] = v;
-            }
-            if (k < NS) {  // over the level this cell read pointwise (no other cell reads it now)
-                if (odd) {
-                    LB[xb][zb] = v;
-                    if constexpr (ADJ) PB[xb][zb] = pv;
-                } else {
-                    LA[xa][za] = v;
-                    if constexpr (ADJ) PA[xa][za] = pv;
-                }
+    for (int s = 0; s < S; ++s) {
+        const int x = xs + s;
+        const bool xing = x >= 0 && x < g.px, xmod = x >= g.nb && x < g.nb + g.nx;
+        u[s] = p[s] = vc[s] = sv[s] = 0.f;
+        fx[s] = 1.f;
+        if (xing) {
+            fx[s] = a.sfx[2 * x] * a.sfx[2 * x + 1];
+            if (zing) {
+                const long long k = (long long)x * g.ldz + z;
+                u[s] = a.X[so + k];
+                p[s] = a.Y[so + k];
+                vc[s] = a.v2[k];
             }
         }
-        if (k < NS) __syncthreads();
+        if (!ADJ && xmod && zmod) sv[s] = a.plane[0][slot * a.pss + (long long)(x - g.nb) * g.nz + zm];
+        mask[s] = zinr && x >= 4 && x < g.px - 4 ? ~0u : 0u;
+    }
+    const int rlane = g.depth - (tz * OZN - G);  // the receiver row's lane
+    const bool rtile = rlane >= 0 && rlane < 64, rown = rlane >= G && rlane < 64 - G;
+    float tv = 0.f;  // adjoint: the strip's injected samples of every step, one per lane
+    if (ADJ && rtile && lane < NS * S) {
+        const int x = xs + lane % S - g.nb;
+        if (x >= 0 && x < g.nx) {
+            const float* r = a.row[0];
+#pragma unroll
+            for (int k = 1; k < NS; ++k) r = lane / S == k ? a.row[k] : r;
+            tv = r[slot * a.rss + x];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+        const int lo = 4 * k, hi = NX - 4 * k;  // columns valid before this step
+        float* row = lds[k & 1] + 4;
+        const bool live = c0 + S > lo + 4 && c0 < hi - 4;
+        float c[S], nsv[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            c[s] = ADJ ? u[s] * vc[s] : u[s];
+            nsv[s] = 0.f;
+        }
+        if (c0 + S > lo && c0 < hi) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) row[(c0 + s) * 64 + lane] = c[s];
+        }
+        if (!ADJ && k + 1 < NS && live) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const int x = xs + s - g.nb;
+                if (x >= 0 && x < g.nx && zmod) nsv[s] = a.plane[k + 1][slot * a.pss + (long long)x * g.nz + zm];
+            }
+        }
+        // what a step records of the level before it: the receiver row, the image
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int x = xs + s - g.nb;
+            if (c0 + s < G || c0 + s >= NX - G || x < 0 || x >= g.nx) continue;
+            if (!ADJ) {
+                if (rown && lane == rlane) a.row[k][slot * a.rss + x] = 0.f + u[s];
+            } else if (zown && zmod) {
+                a.plane[k][slot * a.pss + (long long)x * g.nz + zm] = 0.f + c[s];
+            }
+        }
+        __syncthreads();
+        if (!live) continue;
+        // the strip's columns and four on either side (the tile's edge strips read any column there)
+        float q[S + 8];
+        const int cl = max(c0 - 4, 0), cr = min(c0 + S, NX - 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            q[i] = row[(cl + i) * 64 + lane];
+            q[S + 4 + i] = row[(cr + i) * 64 + lane];
+        }
+        float zn[S][8];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float* R = row + (c0 + s) * 64 + lane;
+            q[s + 4] = c[s];
+#pragma unroll
+            for (int i = 1; i <= 4; ++i) {
+                zn[s][i - 1] = R[-i];
+                zn[s][i + 3] = R[i];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every LDS read in flight before the first wait
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float lx = W4 * (q[s + 8] + q[s]) + W3 * (q[s + 7] + q[s + 1]) + W2 * (q[s + 6] + q[s + 2]) +
+                             W1 * (q[s + 5] + q[s + 3]) + W0 * q[s + 4];
+            const float lz = W4 * (zn[s][7] + zn[s][3]) + W3 * (zn[s][6] + zn[s][2]) + W2 * (zn[s][5] + zn[s][1]) +
+                             W1 * (zn[s][4] + zn[s][0]) + W0 * q[s + 4];
+            const float l = lx * g.sx + lz * g.sz;
+            float u2 = (ADJ ? l : l * vc[s]) + 2.0f * u[s] - fx[s] * (fz * p[s]);
+            u2 = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, u2) & mask[s]);
+            const int x = xs + s - g.nb;
+            const bool xmod = x >= 0 && x < g.nx;
+            if (!ADJ) {
+                if (xmod && zmod) u2 = u2 + sv[s] * vc[s];
+            } else if (rtile && xmod) {
+                const float v = __shfl(tv, k * S + s);
+                if (lane == rlane) u2 = u2 + v;
+            }
+            p[s] = u[s];
+            u[s] = fx[s] * (fz * u2);
+            sv[s] = nsv[s];
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int x = xs + s;
+        if (zown && c0 + s >= G && c0 + s < NX - G && x < g.px) {
+            const long long k = so + (long long)x * g.ldz + z;
+            a.D[k] = u[s];
+            a.C[k] = p[s];
+        }
     }
 }
 
@@ -823,13 +767,13 @@ struct pw_lstri {
     float* fields = nullptr;  // 4 * cap_slots fields (two levels, and two for the two-step launches)
     int cap_slots = 0;
     int spl = 1;              // time steps per sweep launch: 1, 2 or 4
-    int oxn = 4;              // output columns of the four-step launches' tiles (4 or 8)
+    int oxn = 4;              // columns per wave of the four-step launches (4 or 8)
     // launch choice per shots-per-sweep count: {single-step tile width, steps per launch, four-step
-    // tile columns}, from timing both sweeps' launches on the plan's own grid and buffers
+    // columns per wave}, from timing both sweeps' launches on the plan's own grid and buffers
     std::map<int, std::vector<int>> choice;
     int spl_forced = 0;       // 0: the timed choice; 1, 2 or 4 steps per launch
     int xct_forced = 0;       // 0: the timed choice; else this single-step tile width
-    int oxn_forced = 0;       // 0: the timed choice; else the four-step tiles' output columns
+    int oxn_forced = 0;       // 0: the timed choice; else the four-step launches' columns per wave
     std::vector<float> tune_log;  // (kernel, width, ms per launch) of the last timing sweep
     int graph_xct = 0, graph_spl = -1, graph_oxn = 0;  // the launch choice the captured CG sweeps hold
     float *src = nullptr, *dat = nullptr, *stage = nullptr;  // batch buffers (modelling / imaging)
@@ -913,18 +857,19 @@ void step2(pw_lstri* p, bool adj, int nslot, const TriArgs2& a)
 }
 
 // four steps per launch (k_trn): a.X, a.Y in; a.C, a.D out
-void step4(pw_lstri* p, bool adj, int nslot, const TriArgsN<4>& a)
+template <int S>
+void launch_trn(pw_lstri* p, bool adj, int nslot, const TriArgsN<NSN>& a)
 {
-    const int ntz = (p->g.pz + OZN - 1) / OZN, ntx = (p->g.px + p->oxn - 1) / p->oxn;
-    dim3 grid(ntz * ntx, nslot);
-    hipStream_t s = p->ctx->s();
-    if (p->oxn == 8) {
-        if (adj) hipLaunchKernelGGL((k_trn<true, 4, 8>), grid, dim3(TN), 0, s, p->g, a, ntz);
-        else hipLaunchKernelGGL((k_trn<false, 4, 8>), grid, dim3(TN), 0, s, p->g, a, ntz);
-    } else {
-        if (adj) hipLaunchKernelGGL((k_trn<true, 4, 4>), grid, dim3(TN), 0, s, p->g, a, ntz);
-        else hipLaunchKernelGGL((k_trn<false, 4, 4>), grid, dim3(TN), 0, s, p->g, a, ntz);
-    }
+    const int ntz = (p->g.pz + OZN - 1) / OZN, ntx = (p->g.px + trn_owned(S) - 1) / trn_owned(S);
+    const dim3 grid(ntz * ntx, nslot), block(64 * trn_waves(S));
+    if (adj) hipLaunchKernelGGL((k_trn<true, NSN, S>), grid, block, 0, p->ctx->s(), p->g, a, ntz);
+    else hipLaunchKernelGGL((k_trn<false, NSN, S>), grid, block, 0, p->ctx->s(), p->g, a, ntz);
+}
+
+void step4(pw_lstri* p, bool adj, int nslot, const TriArgsN<NSN>& a)
+{
+    if (p->oxn == 8) launch_trn<8>(p, adj, nslot, a);
+    else launch_trn<4>(p, adj, nslot, a);
 }
 
 void step(pw_lstri* p, bool adj, int nslot, const TriArgs& a)
@@ -1519,7 +1464,7 @@ int pw_lstri_steps_per_launch(pw_lstri* p, int n)
     return PW_OK;
 }
 
-// output columns of the four-step launches' tiles: 4, 8, or 0 for the plan's timed choice
+// columns per wave of the four-step launches: 4, 8, or 0 for the plan's timed choice
 int pw_lstri_set_four_step_columns(pw_lstri* p, int c)
 {
     if (!p || !(c == 0 || c == 4 || c == 8)) return PW_ERR_ARG;
@@ -1536,7 +1481,7 @@ int pw_lstri_set_tile_width(pw_lstri* p, int w)
 }
 
 // the launch choice of the last sweep: w[0] single-step tile width, w[1] steps per launch (1, 2, 4),
-// w[2] the four-step tiles' output columns; the timing sweep's (kernel, width, ms per launch)
+// w[2] the four-step launches' columns per wave; the timing sweep's (kernel, width, ms per launch)
 // triples into log[3*cap] (kernel 0 modelling step, 1 adjoint step, 2 two-step modelling, 3
 // two-step adjoint, 4 four-step modelling, 5 four-step adjoint); returns their number
 int pw_lstri_launch_choice(pw_lstri* p, int* w, float* log, int cap)

@@ -102,11 +102,12 @@ class LstriProblem:
         N.check(self._L.pw_lstri_set_tile_width(self._p, int(w)), self._ctx, "set_tile_width")
 
     def set_four_step_columns(self, c=0):
-        """Output columns of the four-step launches' tiles: 4, 8, or 0 for the timed choice."""
+        """Columns per wave of the four-step launches: 4 (tiles of 16 columns), 8 (32), or 0 for the timed
+        choice."""
         N.check(self._L.pw_lstri_set_four_step_columns(self._p, int(c)), self._ctx, "set_four_step_columns")
 
     def launch_choice(self):
-        """(single-step tile width, steps per launch, four-step tile columns) of the last sweep, and
+        """(single-step tile width, steps per launch, four-step columns per wave) of the last sweep, and
         the timing sweep's [(kernel, width, ms per launch), ...]."""
         names = ["model_step", "adjoint_step", "two_step_model", "two_step_adjoint", "four_step_model",
                  "four_step_adjoint"]

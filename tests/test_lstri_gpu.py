@@ -199,3 +199,22 @@ def test_four_step_launches_equal_single_steps(ls, nt, cols):
     assert np.array_equal(a.invert(d4), b.invert(d4))
     with pytest.raises(ValueError):
         b.set_four_step_columns(6)
+
+
+@pytest.mark.parametrize("nz,nx,nb", [(31, 65, 9), (34, 96, 15), (7, 9, 12), (100, 33, 4)])
+@pytest.mark.parametrize("cols", [4, 8])
+def test_four_step_tiles_at_grid_edges_vs_single_steps(nz, nx, nb, cols):
+    # padded grids one cell short of, equal to and beyond whole 32 x 16 and 32 x 32 tiles, the receiver
+    # row in a tile's growth, three shots a launch: the same expressions per cell, so equal
+    rng = np.random.default_rng(nz + nx)
+    nt = 10
+    par = np.array([nz, nx, 0.01, 0.012, 0, 0, nt, 0.001, 0, 0, 3, 0.2, 0, 5, nb, 0.01, 10, 1, 1, 2], np.float32)
+    vel = (1.5 + 2 * rng.random((nz, nx))).astype(np.float32)
+    src = rng.standard_normal((nz, nx, nt, 3)).astype(np.float32)
+    dat = rng.standard_normal((nt, nx, 3)).astype(np.float32)
+    one, four = LstriProblem(par, vel), LstriProblem(par, vel)
+    one.steps_per_launch(1)
+    four.steps_per_launch(4)
+    four.set_four_step_columns(cols)
+    assert np.array_equal(one.model(src), four.model(src))
+    assert np.array_equal(one.image(dat), four.image(dat))
