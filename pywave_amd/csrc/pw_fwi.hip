@@ -2337,6 +2337,13 @@ int tune_widths(pw_fwi* p)
         return PW_OK;
     };
     const bool visco = p->visco && sizeof(T) == 4;
+    // The launches that store or read a step's term take another field of the segment buffer each
+    // time, as a sweep's steps do: timed on one and the same field, which the Infinity Cache then
+    // holds, two exact-adjoint steps per launch measured 70 us for the 400 x 800, 16-shot batch and
+    // were taken against 83 us for two single steps; in the sweep they take 97 against 84.
+    const long long tfld = (long long)p->nslot * p->fs, tslots = std::max(1LL, p->seg_cap / tfld);
+    long long turn = 0;
+    auto term_slot = [&]() { return (T*)p->seg + (turn++ % tslots) * tfld; };
     StepArgs<T> f = base_args<T>(p);
     f.X = (const T*)p->X; f.Y = (T*)p->Y; f.it = 0;
     f.fsrc = step_src<T>(p, 0);
@@ -2353,10 +2360,12 @@ int tune_widths(pw_fwi* p)
         // once): timed on their own, as the extra stream moves the best width
         if (!rc && !p->modelling) {
             StepArgs<T> ft = f;
-            ft.full = (T*)p->seg;
             ft.fulls = p->fs;
             kind = 7;
-            rc = pick([&](int W) { launch_fwd<T, false>(W, g, ft, a.padnz, a.padnx, nb_, s); }, &p->w_fwdt);
+            rc = pick([&](int W) {
+                ft.full = term_slot();
+                launch_fwd<T, false>(W, g, ft, a.padnz, a.padnx, nb_, s);
+            }, &p->w_fwdt);
         }
     }
     if (rc) return rc;
@@ -2394,7 +2403,11 @@ int tune_widths(pw_fwi* p)
     if (!visco) {
         ExArgs<T> ex{(const T*)p->seg, p->fs, (T*)p->gm};
         kind = 2;
-        rc = pick([&](int W) { launch_exact<T>(W, g, b, ex, a.padnz, a.padnx, nb_, s); }, &p->w_exact);
+        auto exact = [&](int W) {
+            ex.F = term_slot();
+            launch_exact<T>(W, g, b, ex, a.padnz, a.padnx, nb_, s);
+        };
+        rc = pick(exact, &p->w_exact);
         if (rc) return rc;
         // two adjoint steps per launch (f32): kept when a launch takes less than two single steps
         p->w_adj2 = 0;
@@ -2405,20 +2418,19 @@ int tune_widths(pw_fwi* p)
                 if (!p->B2 && (rc = dmalloc(p, &p->B2, fld * 4))) return rc;
                 float t1 = 0.f;
                 const int w1 = p->w_exact;
-                if ((rc = time_launches(p, [&] { launch_exact<T>(w1, g, b, ex, a.padnz, a.padnx, nb_, s); }, reps,
-                                        &t1)))
-                    return rc;
-                // the two terms: the first two fields of the segment buffer (it holds K >= 2 of them)
-                const float* F = (const float*)p->seg;
-                const bool two_terms = p->seg_cap >= 2 * fld;
-                Adj2Args<float> r = adj2_args(p, (const float*)p->A, (const float*)p->B, (float*)p->A2,
-                                              (float*)p->B2, F, two_terms ? F + fld : F, a.nt - 1);
+                if ((rc = time_launches(p, [&] { exact(w1); }, reps, &t1))) return rc;
                 float tbest = 0.f;
                 int wbest = 0;
                 for (int W : {8, 16, 32}) {
                     float ms = 0.f;
-                    if ((rc = time_launches(p, [&] { launch_adj2(W, g, r, a.padnz, a.padnx, nb_, s); }, reps, &ms)))
-                        return rc;
+                    auto two = [&] {
+                        const float* F1 = (const float*)term_slot();
+                        const float* F2 = (const float*)term_slot();
+                        const Adj2Args<float> r = adj2_args(p, (const float*)p->A, (const float*)p->B, (float*)p->A2,
+                                                            (float*)p->B2, F1, F2, a.nt - 1);
+                        launch_adj2(W, g, r, a.padnz, a.padnx, nb_, s);
+                    };
+                    if ((rc = time_launches(p, two, reps, &ms))) return rc;
                     note(6, W, ms);
                     if (!wbest || ms < tbest) { tbest = ms; wbest = W; }
                 }
