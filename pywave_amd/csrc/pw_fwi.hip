@@ -1038,6 +1038,231 @@ __global__ __launch_bounds__(64) void k_adj_ref(FGeo<float> g, StepArgs<float> a
     }
 }
 
+// ---------------------------------------------------------------- several steps per launch
+// Small surveys: a single step of one or a few shots on a few hundred cells a side costs the
+// launch and the chain of latencies of one tile (4.7 to 6 us for less than 1 us of traffic).  A
+// block advances the cells it owns K steps of k_fwd or of k_adj_ref.  It holds them grown by 4K
+// cells on every side: lanes run along z (64 - 8K owned), each of W waves owns a strip of S
+// columns, and both levels, v^2dt^2 and the sponge factors stay in registers.  Once per step the
+// strips publish the current level in LDS, read their neighbours along z and across the strip edges
+// and form the new level with the single-step kernels' expressions in their order, so every level,
+// trace, snapshot, term and imaging sum equals single steps bit for bit.  The adjoint leaves the
+// owned cells' levels of its K steps in LDS and images them after the last one, all waves sharing
+// the f64 work, each cell's sum read and written once per launch and consecutive steps sharing
+// their snapshots.  Outputs go to the other pair of fields.
+constexpr int kMulti = 4, kMultiS = 4, kMultiW = 12;  // steps per launch, columns per strip, strips
+
+struct MultiArgs {
+    const float *X, *Y;      // current and previous level
+    float *C, *D;            // out: the last step's previous level, the last step's level
+    const float *m, *sfz, *sfx;
+    const ShotInfo* shots;
+    const float* patch;      // forward: source patches, wavelet, traces out
+    const float* wav;
+    float* rec;
+    const float* inj;        // adjoint: traces in
+    long long trs;
+    float* snap[kMulti];     // forward: interior snapshot per step, or null
+    long long snaps;
+    float* term[kMulti];     // forward: the step's term on the full field, or null
+    long long terms;
+    const float* w0;         // adjoint: the snapshot of step it; step it - k at w0 - k wstep
+    long long wstep;
+    unsigned img;            // bit k: the k-th step of the launch images
+    const float* tmpv;
+    float* grad;
+    long long gstride;
+    int it, nk;              // first step, steps of this launch (adjoint: descending)
+};
+
+template <int K, int S, int W>
+struct MultiTile {
+    static constexpr int halo = 4 * K, owned_z = 64 - 8 * K, cols = S * W, owned_x = cols - 8 * K;
+};
+using FourStep = MultiTile<kMulti, kMultiS, kMultiW>;  // 32 x 16 owned cells
+
+template <bool ADJ, int K, int S, int W>
+__global__ __launch_bounds__(64 * W) void k_multi(FGeo<float> g, MultiArgs a, int ntz)
+{
+    using C = Coef<float>;
+    using M = MultiTile<K, S, W>;
+    constexpr int G = M::halo, NX = M::cols, OZ = M::owned_z, OX = M::owned_x;
+    static_assert(K <= kMulti && K * S <= 64 && OX > 0 && OX * OZ % 64 == 0, "tile");
+    __shared__ float lds[2][NX * 64 + 8];  // four cells of guard at either end
+    __shared__ float lev[ADJ ? K : 1][ADJ ? OX * OZ : 1];  // adjoint: the owned cells' level of each step
+    const int slot = blockIdx.y;
+    const int tz = blockIdx.x % ntz, tx = blockIdx.x / ntz;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int z0 = tz * OZ - G, x0 = tx * OX - G;
+    const int z = z0 + lane, c0 = w * S, xs = x0 + c0;
+    const long long so = (long long)slot * g.fs;
+    const ShotInfo sh = a.shots[slot];
+    const bool zing = z >= 0 && z < g.pnz, zin = z >= 4 && z < g.pnz - 4;
+    const bool zown = zing && lane >= G && lane < 64 - G, zmod = z >= g.nb && z < g.nb + g.nz;
+    const bool sown = c0 + S > G && c0 < NX - G;  // the strip owns columns
+    float u[S], p[S], mv[S], fx[S], pt[S];
+    unsigned mask[S];  // the Laplacian's cells, [4, pad - 4) on both axes
+    const float fz = zing ? a.sfz[2 * z] * a.sfz[2 * z + 1] : 1.f;  // one of a pair is 1
+    const bool hit = !ADJ && sh.pw > 0 && z0 < sh.sz0 + sh.ph && z0 + 64 > sh.sz0 && x0 < sh.sx0 + sh.pw && x0 + NX > sh.sx0;
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int x = xs + s;
+        const bool xing = x >= 0 && x < g.pnx;
+        u[s] = p[s] = mv[s] = pt[s] = 0.f;
+        fx[s] = 1.f;
+        if (xing) {
+            fx[s] = a.sfx[2 * x] * a.sfx[2 * x + 1];
+            if (zing) {
+                const long long k = (long long)x * g.ldz + z;
+                u[s] = a.X[so + k];
+                p[s] = a.Y[so + k];
+                mv[s] = a.m[k];
+            }
+        }
+        if (hit) {
+            const int px = x - sh.sx0, pz = z - sh.sz0;
+            if (px >= 0 && px < sh.pw && pz >= 0 && pz < sh.ph) pt[s] = a.patch[slot * PMAX * PMAX + px * PMAX + pz];
+        }
+        mask[s] = zin && x >= 4 && x < g.pnx - 4 ? ~0u : 0u;
+    }
+    const int rlane = g.rz - z0;  // the receiver row's lane
+    const bool rtile = rlane >= 0 && rlane < 64;
+    float tv = 0.f;  // adjoint: the strip's residual samples of every step, one per lane
+    if (ADJ && rtile && lane < K * S && lane / S < a.nk) {
+        const int d = xs + lane % S - sh.r0_v, k = sh.r02 + d;
+        if (d >= 0 && d < sh.nr2 && k >= 0 && k < g.nr)
+            tv = a.inj[slot * a.trs + (long long)(a.it - lane / S) * g.nr + k];
+    }
+    // adjoint: imaging tasks, 64 owned cells each, dealt over the waves; a task's snapshots
+    // it+1 .. it-K, -2/v^3 and sums are loaded ahead of the steps
+    constexpr int kTasks = OX * OZ / 64, TW = (kTasks + W - 1) / W;
+    float ws[ADJ ? TW : 1][K + 2], tm[ADJ ? TW : 1], gv[ADJ ? TW : 1];
+    auto image_cell = [&](int t, int& e) -> long long {  // the task's cell: index in the model, or -1
+        const int task = w + t * W;
+        e = task * 64 + lane;
+        const int zc = z0 + G + e % OZ - g.nb, xc = x0 + G + e / OZ - g.nb;
+        const bool ok = a.img && task < kTasks && zc >= 0 && zc < g.nz && xc >= 0 && xc < g.nx;
+        return ok ? (long long)xc * g.nz + zc : -1;
+    };
+    if constexpr (ADJ) {
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            int e;
+            const long long c = image_cell(t, e);
+            tm[t] = c >= 0 ? a.tmpv[c] : 0.f;
+            gv[t] = c >= 0 ? a.grad[slot * a.gstride + c] : 0.f;
+#pragma unroll
+            for (int j = 0; j < K + 2; ++j) {
+                const bool need = ((a.img >> j) | (j >= 1 ? a.img >> (j - 1) : 0) | (j >= 2 ? a.img >> (j - 2) : 0)) & 1;
+                ws[t][j] = c >= 0 && need ? a.w0[slot * a.snaps + (1 - j) * a.wstep + c] : 0.f;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (k >= a.nk) break;
+        const int lo = 4 * k, hi = NX - 4 * k;  // columns valid before this step
+        float* row = lds[k & 1] + 4;
+        const bool live = c0 + S > lo + 4 && c0 < hi - 4;
+        if (c0 + S > lo && c0 < hi) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) row[(c0 + s) * 64 + lane] = u[s];
+        }
+        if constexpr (ADJ) {
+            if (sown && a.img) {
+#pragma unroll
+                for (int s = 0; s < S; ++s)
+                    if (c0 + s >= G && c0 + s < NX - G && lane >= G && lane < 64 - G)
+                        lev[k][(c0 + s - G) * OZ + lane - G] = u[s];
+            }
+        }
+        // what a forward step records of the level before it
+        if (!ADJ && sown) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                if (c0 + s < G || c0 + s >= NX - G || !zown) continue;
+                const int d = xs + s - sh.r0_v, kk = sh.r02 + d, x = xs + s - g.nb;
+                if (lane == rlane && d >= 0 && d < sh.nr2 && kk >= 0 && kk < g.nr)
+                    a.rec[slot * a.trs + (long long)(a.it + k) * g.nr + kk] = u[s];
+                if (a.snap[k] && zmod && x >= 0 && x < g.nx)
+                    a.snap[k][slot * a.snaps + (long long)x * g.nz + (z - g.nb)] = u[s];
+            }
+        }
+        __syncthreads();
+        if (!live) continue;
+        // the strip's columns and four on either side (the tile's edge strips read any column there)
+        float q[S + 8], zn[S][8];
+        const int cl = max(c0 - 4, 0), cr = min(c0 + S, NX - 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            q[i] = row[(cl + i) * 64 + lane];
+            q[S + 4 + i] = row[(cr + i) * 64 + lane];
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float* R = row + (c0 + s) * 64 + lane;
+            q[s + 4] = u[s];
+#pragma unroll
+            for (int i = 1; i <= 4; ++i) {
+                zn[s][i - 1] = R[-i];
+                zn[s][i + 3] = R[i];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every LDS read in flight before the first wait
+        const float wv = ADJ ? 0.f : a.wav[a.it + k];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float p1 = q[s + 4];
+            const float lap = (C::K0 * p1 + C::K1 * (q[s + 5] + q[s + 3]) + C::K2 * (q[s + 6] + q[s + 2]) +
+                               C::K3 * (q[s + 7] + q[s + 1]) + C::K4 * (q[s + 8] + q[s])) / g.dx2 +
+                              (C::K0 * p1 + C::K1 * (zn[s][4] + zn[s][0]) + C::K2 * (zn[s][5] + zn[s][1]) +
+                               C::K3 * (zn[s][6] + zn[s][2]) + C::K4 * (zn[s][7] + zn[s][3])) / g.dz2;
+            float term = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, lap) & mask[s]);
+            if (!ADJ) {
+                if (hit) term = term + pt[s] * wv;
+                if (a.term[k] && zown && c0 + s >= G && c0 + s < NX - G && xs + s < g.pnx)
+                    __builtin_nontemporal_store(term, &a.term[k][slot * a.terms + (long long)(xs + s) * g.ldz + z]);
+            } else {
+                if (rtile) {
+                    const float v = __shfl(tv, k * S + s);
+                    const int d = xs + s - sh.r0_v, kk = sh.r02 + d;
+                    if (lane == rlane && d >= 0 && d < sh.nr2 && kk >= 0 && kk < g.nr) term = term + v;
+                }
+            }
+            const float p0 = fx[s] * (fz * p[s]);
+            const float p2 = 2 * p1 - p0 + mv[s] * term;
+            p[s] = u[s];
+            u[s] = fx[s] * (fz * p2);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int x = xs + s;
+        if (!zown || c0 + s < G || c0 + s >= NX - G || x >= g.pnx) continue;
+        const long long k = so + (long long)x * g.ldz + z;
+        a.D[k] = u[s];
+        a.C[k] = p[s];
+    }
+    if constexpr (ADJ) {
+        if (!a.img) return;
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            int e;
+            const long long c = image_cell(t, e);
+            if (c < 0) continue;
+#pragma unroll
+            for (int k = 0; k < K; ++k)
+                if ((a.img >> k) & 1) {
+                    const double v = ((double)ws[t][k] - 2. * (double)ws[t][k + 1] + (double)ws[t][k + 2]) / g.wdt2 *
+                                     (double)lev[k][e] * (double)tm[t];
+                    gv[t] = (float)((double)gv[t] + v);
+                }
+            a.grad[slot * a.gstride + c] = gv[t];
+        }
+    }
+}
+
 // ---------------------------------------------------------------- exact discrete adjoint
 // q_t = S(2 q_{t+1} - S q_{t+2} + L^T(m q_{t+1}) + R^T g_t);  dJ/dm += (L X_t + r w_t) q_{t+1}
 template <typename T>
@@ -2249,6 +2474,68 @@ bool fused2(const pw_fwi* p) { return p->max_fused >= 2 && p->w_fwd2 > 0 && !p->
 // whether exact-adjoint sweeps advance two steps per launch (f32 plans)
 bool fused2_adj(const pw_fwi* p) { return p->max_fused >= 2 && p->w_adj2 > 0 && p->prec == 4 && p->A2; }
 
+// Whether the plan's forward and reference-adjoint sweeps advance kMulti steps per launch: f32
+// acoustic plans with point sources and receivers one cell apart (what pfwi's geometry gives),
+// unless the caller asked for one step per launch, two, or fixed tile widths, while the tiles fit
+// the chip at once (two blocks on each of 256 CUs).  Measured, us per step, multi-step against the
+// fastest single steps, forward / reference adjoint, model and shots (tiles):
+//   60 x 80, 1 (78)       2.67 / 2.75   4.80 / 5.72
+//   101 x 203, 1 (147)    2.75 / 2.90   4.80 / 6.03
+//   101 x 203, 3 (441)    3.85 / 4.82   5.22 / 6.20
+//   200 x 300, 2 (540)    5.10 / 5.35   5.20 / 6.12
+//   400 x 800, 1 (986)    6.55 / 9.32   5.83 / 7.00
+// (Two steps per launch in tiles of 48 x 32 reached 4.5 forward on 200 x 300, 2 shots, and lost
+// everywhere else.)
+bool multi_ok(const pw_fwi* p)
+{
+    const Acq& a = p->acq;
+    const long long tiles = (long long)pw::ceil_div(a.padnz, FourStep::owned_z) *
+                            pw::ceil_div(a.padnx, FourStep::owned_x) * p->nslot;
+    return p->prec == 4 && !p->visco && !p->passive && p->max_fused >= 2 && !p->force_fused && !p->widths_forced &&
+           a.dr_v == 1 && tiles <= 512;
+}
+
+MultiArgs multi_args(pw_fwi* p, const float* X, const float* Y, float* C, float* D, int it, int nk)
+{
+    MultiArgs r{};
+    r.X = X; r.Y = Y; r.C = C; r.D = D;
+    r.m = (const float*)p->m;
+    r.sfz = (const float*)p->sfz;
+    r.sfx = (const float*)p->sfx;
+    r.shots = p->shots;
+    r.patch = (const float*)p->patch;
+    r.wav = (const float*)p->wav;
+    r.trs = (long long)p->acq.nt * p->acq.nr;
+    r.snaps = p->nzx;
+    r.terms = p->fs;
+    r.it = it;
+    r.nk = nk;
+    return r;
+}
+
+int launch_multi(pw_fwi* p, bool adj, const MultiArgs& r, int nb_)
+{
+    const Acq& a = p->acq;
+    const int ntz = pw::ceil_div(a.padnz, FourStep::owned_z);
+    const dim3 grid(ntz * pw::ceil_div(a.padnx, FourStep::owned_x), nb_), block(64 * kMultiW);
+    const FGeo<float> g = geo<float>(p);
+    if (adj) hipLaunchKernelGGL((k_multi<true, kMulti, kMultiS, kMultiW>), grid, block, 0, p->ctx->s(), g, r, ntz);
+    else hipLaunchKernelGGL((k_multi<false, kMulti, kMultiS, kMultiW>), grid, block, 0, p->ctx->s(), g, r, ntz);
+    PW_HIPS(hipGetLastError());
+    return PW_OK;
+}
+
+// the second pair of forward (adj: adjoint) fields, allocated when a sweep first needs it
+int multi_fields(pw_fwi* p, bool adj)
+{
+    const size_t bytes = (size_t)p->nslot * p->fs * 4;
+    void** f[2] = {adj ? (void**)&p->A2 : (void**)&p->X2, adj ? (void**)&p->B2 : (void**)&p->Y2};
+    for (void** q : f)
+        if (!*q)
+            if (int rc = dmalloc(p, q, bytes)) return rc;
+    return PW_OK;
+}
+
 Adj2Args<float> adj2_args(pw_fwi* p, const float* A, const float* B, float* C, float* D, const float* F1,
                           const float* F2, int it)
 {
@@ -2525,7 +2812,9 @@ int forward_batch(pw_fwi* p, int nb_, bool ckpt, int mode, bool store_last)
     }
     const int I = a.interval, K = p->K;
     const int last = p->nseg - 1, a_last = last * K;
-    T* Sa = (T*)p->X2;  // the two-step launches' output fields
+    const bool multi = sizeof(T) == 4 && multi_ok(p);
+    if (multi && (rc = multi_fields(p, false))) return rc;
+    T* Sa = (T*)p->X2;  // the multi-step launches' output fields
     T* Sb = (T*)p->Y2;
     // what step it stores besides its level: an interior snapshot, or its term (exact adjoint)
     auto io = [&](int it, T** snap, T** full) {
@@ -2547,6 +2836,20 @@ int forward_batch(pw_fwi* p, int nb_, bool ckpt, int mode, bool store_last)
             PW_HIPS(hipMemcpyAsync(c + fld, Y, fld * sizeof(T), hipMemcpyDeviceToDevice, s));
             if (visco)  // the memory variable of the same level as X
                 PW_HIPS(hipMemcpyAsync(p->ckpt_r + (size_t)sgi * fld, Ra, fld * 4, hipMemcpyDeviceToDevice, s));
+        }
+        if constexpr (sizeof(T) == 4) {
+            if (multi) {  // up to kMulti steps, to the next checkpoint or the end
+                int nk = std::min(kMulti, a.nt - it);
+                if (ckpt) nk = std::min(nk, (it / K + 1) * K - it);
+                MultiArgs r = multi_args(p, X, Y, Sa, Sb, it, nk);
+                r.rec = (float*)p->rec;
+                for (int k = 0; k < nk; ++k) io(it + k, &r.snap[k], &r.term[k]);
+                if ((rc = launch_multi(p, false, r, nb_))) return rc;
+                std::swap(X, Sb);
+                std::swap(Y, Sa);
+                it += nk;
+                continue;
+            }
         }
         // two steps in one launch unless a checkpoint falls between them
         if (fused2(p) && it + 1 < a.nt && !(ckpt && (it + 1) % K == 0)) {
@@ -2706,7 +3009,35 @@ int adjoint_segment(pw_fwi* p, int nb_, int sg, int mode, T** Ap, T** Bp, T* gra
         PW_HIPS(hipMemcpyAsync(p->seg, (T*)p->ckpt_snap + (size_t)sg * p->nslot * p->nzx,
                                (size_t)p->nslot * p->nzx * sizeof(T), hipMemcpyDeviceToDevice, s));
     }
-    for (int it = b0 - 1; it >= a0; --it) {
+    int it = b0 - 1;
+    if constexpr (sizeof(T) == 4) {
+        if (mode == 0 && I == 1 && multi_ok(p)) {
+            if (int rc = multi_fields(p, true)) return rc;
+            if (!p->adj_sa) { p->adj_sa = p->A2; p->adj_sb = p->B2; }
+            float* Sa = (float*)p->adj_sa;
+            float* Sb = (float*)p->adj_sb;
+            const long long ss = (long long)p->nslot * p->nzx;
+            while (it >= a0) {
+                const int nk = std::min(kMulti, it - a0 + 1);
+                MultiArgs r = multi_args(p, A, B, Sa, Sb, it, nk);
+                r.inj = (const float*)p->res;
+                r.w0 = (const float*)p->seg + (size_t)(it - a0 + 1) * ss;
+                r.wstep = ss;
+                for (int k = 0; k < nk; ++k)
+                    if (it - k != wnt - 1 && it - k != 0) r.img |= 1u << k;
+                r.tmpv = p->tmpv;
+                r.grad = grad_ref;
+                r.gstride = gstride;
+                if (int rc = launch_multi(p, true, r, nb_)) return rc;
+                std::swap(A, Sb);
+                std::swap(B, Sa);
+                it -= nk;
+            }
+            p->adj_sa = Sa;
+            p->adj_sb = Sb;
+        }
+    }
+    for (; it >= a0; --it) {
         StepArgs<T> s_ = base_args<T>(p);
         s_.X = A; s_.Y = B; s_.it = it;
         s_.fsrc = step_src<T>(p, it);

@@ -358,3 +358,27 @@ def test_forced_widths_give_the_reference_results(small):
         p.close()
     with pytest.raises(ValueError):
         FwiProblem(small["par"], small["wav"], batch=1).set_widths(forward=5)
+
+
+@pytest.mark.parametrize("nz,nx,ns,nb,nt,ckpt,acqui", [(40, 72, 2, 12, 61, 0, 1), (9, 200, 1, 4, 30, 7, 1),
+                                                       (66, 30, 3, 15, 22, 4, 2), (130, 131, 5, 33, 11, 130, 1)])
+def test_four_step_launches_equal_single_steps(nz, nx, ns, nb, nt, ckpt, acqui):
+    # padded grids around whole 32 x 16 tiles, run lengths and segments that leave one to three
+    # steps in the last launch, receivers fixed and moving with the source: data, misfit and the
+    # imaging gradient (one shot per launch and all together) equal the one-step launches bit for bit
+    rng = np.random.default_rng(nz + nx + nt)
+    par = dict(nz=nz, nx=nx, dz=0.01, dx=0.012, oz=0, ox=0, ns=ns, ds=0.036, os=0.06, sz=5, nt=nt, dt=0.001, ot=0,
+               nb=nb, coef=0.005, acqui_type=acqui, interval=1, f0=10, inv=0, niter=2)
+    vel = (1.5 + 1.5 * rng.random((nz, nx))).astype(np.float32)
+    wav = (1e6 * rng.standard_normal(nt)).astype(np.float32)
+    obs = rng.standard_normal((nt, nx, ns)).astype(np.float32)
+    for batch in (0, 1):
+        out = []
+        for steps in (2, 1):
+            p = FwiProblem(par, wav, data=obs, batch=batch, checkpoint=ckpt)
+            p.set_steps_per_launch(steps)
+            out.append((p.forward(vel),) + p.gradient(vel, "reference"))
+            p.close()
+        (d4, g4, f4, s4), (d1, g1, f1, s1) = out
+        assert np.array_equal(d4, d1) and d1.any()
+        assert np.array_equal(g4, g1) and f4 == f1 and s4 == s1
