@@ -1456,6 +1456,138 @@ __global__ __launch_bounds__(64) void k_adj_exact(FGeo<T> g, StepArgs<T> a, ExAr
     }
 }
 
+// ---------------------------------------------------------------- exact adjoint, several steps per launch
+// k_adj_exact's steps it, it - 1, ... (nk <= K of them) in k_multi's tiles and strips: the product
+// m q, zero outside [4, pad - 4), is what the strips publish, dJ/dm of an owned cell stays in a
+// register over the launch, and the terms of its K steps are loaded ahead of them.  Contracted to
+// FMAs with reciprocal spacings like k_adj_exact (f32 rounding differs from it in the last place).
+// Measured, us per step against the fastest single steps: 60 x 80, 1 shot 2.2 against 5.25;
+// 101 x 203, 3 shots 3.7 against 6.2.
+struct MultiExact {
+    const float *X, *Y;      // q_{it+1}, q_{it+2}
+    float *C, *D;            // out: the last step's previous level, the last step's level
+    const float *m, *sfz, *sfx;
+    const ShotInfo* shots;
+    const float* inj;
+    long long trs;
+    const float* F;          // term of step it; of step it - k at F - k fstep, slot stride fsl
+    long long fstep, fsl;
+    float* gm;
+    int it, nk;
+};
+
+template <int K, int S, int W>
+__global__ __launch_bounds__(64 * W) void k_multi_exact(FGeo<float> g, MultiExact a, int ntz)
+{
+#pragma clang fp contract(fast)
+    using C = Coef<float>;
+    using M = MultiTile<K, S, W>;
+    constexpr int G = M::halo, NX = M::cols;
+    __shared__ float lds[2][NX * 64 + 8];  // four cells of guard at either end
+    const int slot = blockIdx.y;
+    const int tz = blockIdx.x % ntz, tx = blockIdx.x / ntz;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int z0 = tz * M::owned_z - G, x0 = tx * M::owned_x - G;
+    const int z = z0 + lane, c0 = w * S, xs = x0 + c0;
+    const long long so = (long long)slot * g.fs;
+    const ShotInfo sh = a.shots[slot];
+    const float rdx = 1.f / g.dx2, rdz = 1.f / g.dz2;
+    const bool zing = z >= 0 && z < g.pnz, zin = z >= 4 && z < g.pnz - 4;
+    const bool zown = zing && lane >= G && lane < 64 - G;
+    float u[S], p[S], mv[S], fx[S], gv[S], ts[K][S];
+    unsigned on[S];  // cells of the grid
+    const float fz = zing ? a.sfz[2 * z] * a.sfz[2 * z + 1] : 1.f;  // one of a pair is 1
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int x = xs + s;
+        const bool xing = x >= 0 && x < g.pnx;
+        const long long k = (long long)x * g.ldz + z;
+        u[s] = p[s] = mv[s] = gv[s] = 0.f;
+        fx[s] = 1.f;
+        if (xing) {
+            fx[s] = a.sfx[2 * x] * a.sfx[2 * x + 1];
+            if (zing) {
+                u[s] = a.X[so + k];
+                p[s] = a.Y[so + k];
+                if (zin && x >= 4 && x < g.pnx - 4) mv[s] = a.m[k];  // zero off the Laplacian's cells
+            }
+        }
+        on[s] = zing && xing ? ~0u : 0u;
+        const bool own = zown && xing && c0 + s >= G && c0 + s < NX - G;
+        if (own) gv[s] = a.gm[so + k];
+#pragma unroll
+        for (int j = 0; j < K; ++j)
+            ts[j][s] = own && j < a.nk ? __builtin_nontemporal_load(&a.F[slot * a.fsl - j * a.fstep + k]) : 0.f;
+    }
+    const int rlane = g.rz - z0;  // the receiver row's lane
+    const bool rtile = rlane >= 0 && rlane < 64;
+    float tv = 0.f;  // the strip's trace samples of every step, one per lane
+    if (rtile && lane < K * S && lane / S < a.nk) {
+        const int d = xs + lane % S - sh.r0_v, k = sh.r02 + d;
+        if (d >= 0 && d < sh.nr2 && k >= 0 && k < g.nr)
+            tv = a.inj[slot * a.trs + (long long)(a.it - lane / S) * g.nr + k];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        if (k >= a.nk) break;
+        const int lo = 4 * k, hi = NX - 4 * k;  // columns valid before this step
+        float* row = lds[k & 1] + 4;
+        float c[S];
+#pragma unroll
+        for (int s = 0; s < S; ++s) c[s] = mv[s] * u[s];
+        if (c0 + S > lo && c0 < hi) {
+#pragma unroll
+            for (int s = 0; s < S; ++s) row[(c0 + s) * 64 + lane] = c[s];
+        }
+        __syncthreads();
+        if (c0 + S <= lo + 4 || c0 >= hi - 4) continue;
+        // the strip's columns and four on either side (the tile's edge strips read any column there)
+        float q[S + 8], zn[S][8];
+        const int cl = max(c0 - 4, 0), cr = min(c0 + S, NX - 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            q[i] = row[(cl + i) * 64 + lane];
+            q[S + 4 + i] = row[(cr + i) * 64 + lane];
+        }
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float* R = row + (c0 + s) * 64 + lane;
+            q[s + 4] = c[s];
+#pragma unroll
+            for (int i = 1; i <= 4; ++i) {
+                zn[s][i - 1] = R[-i];
+                zn[s][i + 3] = R[i];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every LDS read in flight before the first wait
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const float lt = (C::K0 * q[s + 4] + C::K1 * (q[s + 5] + q[s + 3]) + C::K2 * (q[s + 6] + q[s + 2]) +
+                              C::K3 * (q[s + 7] + q[s + 1]) + C::K4 * (q[s + 8] + q[s])) * rdx +
+                             (C::K0 * q[s + 4] + C::K1 * (zn[s][4] + zn[s][0]) + C::K2 * (zn[s][5] + zn[s][1]) +
+                              C::K3 * (zn[s][6] + zn[s][2]) + C::K4 * (zn[s][7] + zn[s][3])) * rdz;
+            float qn = 2 * u[s] - fx[s] * (fz * p[s]) + lt;
+            qn = __builtin_bit_cast(float, __builtin_bit_cast(unsigned, qn) & on[s]);
+            if (rtile) {
+                const float v = __shfl(tv, k * S + s);
+                if (lane == rlane) qn = qn + v;  // 0 off the receivers
+            }
+            gv[s] = gv[s] + ts[k][s] * u[s];
+            p[s] = u[s];
+            u[s] = fx[s] * (fz * qn);
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) {
+        const int x = xs + s;
+        if (!zown || c0 + s < G || c0 + s >= NX - G || x >= g.pnx) continue;
+        const long long k = so + (long long)x * g.ldz + z;
+        a.D[k] = u[s];
+        a.C[k] = p[s];
+        a.gm[k] = gv[s];
+    }
+}
+
 // ---------------------------------------------------------------- exact adjoint, two steps per launch
 // Temporal blocking of k_adj_exact for batched sweeps (f32): one launch takes (q_{t+1}, q_{t+2}) to
 // (q_{t-1}, q_t), written to two other buffers, and adds both steps' dJ/dm terms in one
@@ -2474,7 +2606,7 @@ bool fused2(const pw_fwi* p) { return p->max_fused >= 2 && p->w_fwd2 > 0 && !p->
 // whether exact-adjoint sweeps advance two steps per launch (f32 plans)
 bool fused2_adj(const pw_fwi* p) { return p->max_fused >= 2 && p->w_adj2 > 0 && p->prec == 4 && p->A2; }
 
-// Whether the plan's forward and reference-adjoint sweeps advance kMulti steps per launch: f32
+// Whether the plan's forward and adjoint sweeps advance kMulti steps per launch: f32
 // acoustic plans with point sources and receivers one cell apart (what pfwi's geometry gives),
 // unless the caller asked for one step per launch, two, or fixed tile widths, while the tiles fit
 // the chip at once (two blocks on each of 256 CUs).  Measured, us per step, multi-step against the
@@ -2989,11 +3121,41 @@ int adjoint_segment2(pw_fwi* p, int nb_, int sg, float** Ap, float** Bp)
     return PW_OK;
 }
 
+// exact-adjoint sweep of segment sg in launches of up to kMulti steps (k_multi_exact)
+int adjoint_segment_multi(pw_fwi* p, int nb_, int sg, float** Ap, float** Bp)
+{
+    const Acq& a = p->acq;
+    if (int rc = multi_fields(p, true)) return rc;
+    if (!p->adj_sa) { p->adj_sa = p->A2; p->adj_sb = p->B2; }
+    float *A = *Ap, *B = *Bp, *Sa = (float*)p->adj_sa, *Sb = (float*)p->adj_sb;
+    const long long fld = (long long)p->nslot * p->fs;
+    const int a0 = sg * p->K, b0 = std::min(a0 + p->K, a.nt);
+    const int ntz = pw::ceil_div(a.padnz, FourStep::owned_z);
+    const dim3 grid(ntz * pw::ceil_div(a.padnx, FourStep::owned_x), nb_), block(64 * kMultiW);
+    for (int it = b0 - 1; it >= a0;) {
+        const int nk = std::min(kMulti, it - a0 + 1);
+        const MultiExact r{A, B, Sa, Sb, (const float*)p->m, (const float*)p->sfz, (const float*)p->sfx, p->shots,
+                           (const float*)p->res, (long long)a.nt * a.nr, (const float*)p->seg + (size_t)(it - a0) * fld,
+                           fld, p->fs, (float*)p->gm, it, nk};
+        hipLaunchKernelGGL((k_multi_exact<kMulti, kMultiS, kMultiW>), grid, block, 0, p->ctx->s(), geo<float>(p), r, ntz);
+        PW_HIPS(hipGetLastError());
+        std::swap(A, Sb);
+        std::swap(B, Sa);
+        it -= nk;
+    }
+    *Ap = A;
+    *Bp = B;
+    p->adj_sa = Sa;
+    p->adj_sb = Sb;
+    return PW_OK;
+}
+
 // backward sweep for segment sg: steps b0-1 .. a0
 template <typename T>
 int adjoint_segment(pw_fwi* p, int nb_, int sg, int mode, T** Ap, T** Bp, T* grad_ref, long long gstride)
 {
     if constexpr (sizeof(T) == 4) {
+        if (mode == 1 && multi_ok(p)) return adjoint_segment_multi(p, nb_, sg, Ap, Bp);
         if (mode == 1 && fused2_adj(p)) return adjoint_segment2(p, nb_, sg, Ap, Bp);
     }
     const Acq& a = p->acq;
