@@ -367,11 +367,12 @@ def lstri_bench():
 def aps3d_bench(cpu_steps=20):
     """Pseudo-spectral 3D modelling on the reference demo's configuration (demos/test_first.py:
     81^3 at 20 m, v = 1500 + 24 z m/s, nbt=30 -> 141^3 updated, 144^3 padded FFT grid, nt=1501,
-    aps3d's default three sources).  Per step: real z transforms, x and y transforms (the y pass
-    fused with the wavenumber multiply and its inverse), inverse x and z, then the leapfrog update.
-    Bytes per step and padded cell as the passes move them: z forward 8, x forward 16, y fused 20,
-    x inverse 16, z inverse 12 (f32 in, complex half-spectrum out and back), update 20 per updated
-    cell (u_n, u_{n-1}, vv, Laplacian read; u_{n+1} written)."""
+    aps3d's default three sources).  Per step: x and y transforms (the y pass fused with the
+    wavenumber multiply and its inverse), inverse x, and one pass over z columns (inverse transform,
+    leapfrog update, the new field's forward transform).
+    Bytes per step as the passes move them: x forward 16 per bin of the half spectrum (complex in
+    and out), y fused 20 (the operator too), x inverse 16, z columns 16 per bin and 16 per updated
+    cell (u_n, u_{n-1}, vv read; u_{n+1} written)."""
     from pywave_amd import AfdPlan
 
     n, nbt, nt, dt, d = 81, 30, 1501, 0.001, 20.0
@@ -388,10 +389,8 @@ def aps3d_bench(cpu_steps=20):
     m = n + 2 * nbt
     n1 = n2 = n3 = 144
     nk = n1 // 2 + 1
-    cells_p = n1 * n2 * n3
     spec = nk * n2 * n3 * 8.0  # bytes of the half spectrum
-    step_bytes = (4.0 * cells_p + spec) + 2 * spec + (2 * spec + 4.0 * nk * n2 * n3) + 2 * spec + \
-                 (spec + 4.0 * cells_p) + 20.0 * m ** 3
+    step_bytes = 8 * spec + 4.0 * nk * n2 * n3 + 16.0 * m ** 3
     step_us = ms * 1e3 / nt
     res = {"workload": "aps3d 81^3 at 20 m (+30 ABC: 141^3, FFT grid 144^3), nt=1501, 3 sources (demos/test_first.py)",
            "run_ms": round(ms, 2), "step_us": round(step_us, 2),

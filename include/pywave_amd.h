@@ -197,9 +197,10 @@ int pw_fwi_adjoint_dev(pw_fwi *p, const void *d_vel, const void *d_gtraces, void
  * exact adjoint; w[8] the width of forward steps that store their term for the exact adjoint
  * (9 ints) */
 int pw_fwi_widths(pw_fwi *p, int *w);
-/* forward time steps one launch may advance: 2 (default; the plan's timing sweep keeps two steps
- * per launch where they are faster), 1 (one kernel per time step, the plain method) or -2 (two
- * steps per launch whatever the timing; acoustic point-source plans) */
+/* time steps one launch may advance: 2 (default: four on acoustic point-source plans small enough
+ * that all their tiles fit the chip at once, else two where the plan's timing sweep finds them
+ * faster), 1 (one kernel per time step, the plain method) or -2 (two steps per launch whatever the
+ * timing; acoustic point-source plans) */
 int pw_fwi_set_steps_per_launch(pw_fwi *p, int n);
 /* force the step kernels' tile widths instead of timing them: w[0] forward, w[1] visco forward,
  * w[2] exact adjoint, w[3] reference adjoint, w[4] visco reference adjoint, each 4, 8 or 16 (one

@@ -1,4 +1,4 @@
-// pw_afd.hip -- afd2d/afd3d on MI355X: one fused kernel per time step.
+// pw_afd.hip -- afd2d/afd3d on MI355X: one fused kernel per time step (3D) or per four to eight (2D).
 //
 // Reference path: pywave/src/wave_fdm.c:397-686 (fdm2d) and :28-381 (fdm), set up by
 // pywave/src/afd.c:23-578.  Per step the reference does, in separate passes,

@@ -1,4 +1,4 @@
-// pw_afd2d.h -- several time steps of the 2D acoustic engine per launch (pw_afd.hip, pw_batch.hip).
+// pw_afd2d.h -- several time steps of the 2D acoustic engine per launch (pw_afd.hip).
 //
 // fdm2d's step (pywave/src/wave_fdm.c:551-662) reads C_n and C_{n-1} and writes C_{n+1}; one step
 // per launch moves 16 B a cell and, on grids of a few hundred cells a side, costs mostly the

@@ -635,8 +635,8 @@ PsLap* ps_create(int n1, int n2, int n3, int ldz, long long ldxy, float dz, floa
         err = "spectral Laplacian: bad padded extents";
         return nullptr;
     }
-    // z lines to 4680 samples, x and y lines to 1820 points: one line takes 24 B of LDS a point (z:
-    // a pair of samples) in k_ps_line and k_ps_z
+    // z lines to 4680 samples, x and y lines to 1820 points: one line takes 24 B of LDS a point in
+    // k_ps_line and 44 B a pair of samples in k_ps_z (103 KB at the longest)
     if (n1 > 4680 || std::max(n2, n3) > 1820) {
         err = "spectral Laplacian: a transform line exceeds the 64 KB of LDS per workgroup";
         return nullptr;

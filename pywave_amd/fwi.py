@@ -155,9 +155,10 @@ class FwiProblem:
         N.check(self._L.pw_fwi_set_widths(self._p, N.ptr(w)), self._ctx, "set_widths")
 
     def set_steps_per_launch(self, n):
-        """Forward time steps one launch may advance: 2 (default: two-step launches where the plan's
-        timing sweep finds them faster), 1 (one kernel per time step, the plain method) or -2 (two
-        steps per launch whatever the timing, on acoustic point-source plans)."""
+        """Time steps one launch may advance: 2 (default: four-step launches on acoustic point-source
+        plans small enough that all their tiles fit the chip at once, else two-step launches where
+        the plan's timing sweep finds them faster), 1 (one kernel per time step, the plain method) or
+        -2 (two steps per launch whatever the timing, on acoustic point-source plans)."""
         N.check(self._L.pw_fwi_set_steps_per_launch(self._p, int(n)), self._ctx, "set_steps_per_launch")
 
     def timing(self):
