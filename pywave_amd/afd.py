@@ -11,7 +11,8 @@ Same signatures, argument meaning and return conventions as the reference wrappe
     ignores the rest);
   * a velocity length that does not match nz*nx[*ny] raises SystemError, as the reference's
     NULL return without an exception does (pywave/src/afd.c:89-93,381-385).
-The engine itself runs as one fused HIP kernel per time step (pywave_amd/csrc/pw_afd.hip).
+The engine itself runs as one fused HIP kernel per 3D time step, or per four to eight 2D steps
+(pywave_amd/csrc/pw_afd.hip).
 """
 import ctypes
 

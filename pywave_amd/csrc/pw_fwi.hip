@@ -9,7 +9,7 @@
 //   smoothing         pywave/src/wave_fwiutil.c:298-335 (gradient_smooth2)
 //   optimiser         pywave/src/wave_fwi.c:24-119, pywave/src/wave_fwilbfgs.c:9-165
 //
-// One fused kernel per time step and shot batch.  As in the afd engine the reference's separate
+// One fused kernel per time step and shot batch (small surveys: per four steps).  As in the afd engine the reference's separate
 // passes (record, snapshot, Laplacian, source add, leapfrog, rotate, sponge both levels) become
 // one pass per cell: the kernel reads p1 (sponged) and the previous p1 (sponged once), forms the
 // second sponge of p0 on read, writes S(2 p1 - S(p0raw) + (v v dt^2)(lap p1 + rr w)) over p0raw.
