@@ -638,7 +638,16 @@ PsLap* ps_create(int n1, int n2, int n3, int ldz, long long ldxy, float dz, floa
     // z lines to 4680 samples, x and y lines to 1820 points: one line takes 24 B of LDS a point in
     // k_ps_line and 44 B a pair of samples in k_ps_z (103 KB at the longest)
     if (n1 > 4680 || std::max(n2, n3) > 1820) {
-        err = "spectral Laplacian: a transform line exceeds the 64 KB of LDS per workgroup";
+        err = "spectral Laplacian: transform lines may have up to 4680 samples along z and 1820 along x and y, not " +
+              std::to_string(n1) + " x " + std::to_string(n2) + " x " + std::to_string(n3);
+        return nullptr;
+    }
+    // 1/(n1 n2 n3) takes the cell count in int, and the lines' element offsets are 32-bit: below 2^31
+    // cells there are fewer than 2^31 bins, the padding of the columns to 16 bins included (at most
+    // 2^30 + 16 * 1820^2)
+    if ((long long)n1 * n2 * n3 >= 1LL << 31) {
+        err = "spectral Laplacian: the padded grid " + std::to_string(n1) + " x " + std::to_string(n2) + " x " +
+              std::to_string(n3) + " holds 2^31 cells or more";
         return nullptr;
     }
     PsLap* P = new PsLap;

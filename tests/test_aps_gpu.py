@@ -10,6 +10,7 @@ import pytest
 import pywave_amd
 from oracle import oracle as O
 from pywave_amd import AfdPlan
+from pywave_amd import _native as N
 
 pytestmark = pytest.mark.gpu
 
@@ -122,3 +123,18 @@ def test_aps3d_lines_per_block_vs_oracle(shape):
     assert np.array_equal(out[:n].reshape(nt, nx, ny, order="F"), d.transpose(2, 1, 0))
     w = out[n:].reshape(nz, nx, ny, -1, order="F")
     assert all(np.array_equal(w[..., k], snaps[k].transpose(2, 1, 0)) for k in range(w.shape[-1]))
+
+
+@pytest.mark.parametrize("shape,what", [((4000, 740, 740), "2^31 cells"), ((4700, 3, 3), "4680 samples"),
+                                        ((8, 1830, 3), "1820 along x and y"), ((8, 3, 1830), "1820 along x and y")])
+def test_spectral_extents_refused(shape, what):
+    # padded grids of 2^31 cells or more (2.25e9 here) and lines beyond the kernels' lengths: refused
+    # when the plan becomes spectral, before the operator is formed
+    L, ctx = N.lib(), N.context()
+    p = L.pw_afd_create(ctx, 3, *shape, 10.0, 10.0, 10.0, 1, 0.001, 0, 0.01, 0)
+    assert p
+    try:
+        assert L.pw_afd_set_spectral(p, 1) == -1
+        assert what in L.pw_last_error(ctx).decode()
+    finally:
+        L.pw_afd_destroy(p)
