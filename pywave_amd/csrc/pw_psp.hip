@@ -576,6 +576,13 @@ size_t line_lds(int n, int lpb, bool both) { return ((size_t)(both ? 2 : 1) * lp
 // k_ps_z: two line buffers, twiddles, super-twiddles, damping pairs
 size_t z_lds(int h, int lpb) { return (((size_t)2 * z_stride(lpb) + 3) * h + (h + 1) / 2) * sizeof(cf); }
 
+// A line or z column that has a block to itself gets 256 threads, a z column of more than kLongColumn
+// pairs (whose LDS leaves at most three blocks on a CU) 512.  Measured, us a step with 64, 256 and
+// 512 threads (two kernels of whole lines, 256 threads, before): 2D 181 x 227 cells 17.9, 17.2 and
+// 16.9 (36.7), 960^2 65, 44 and 50 (56), 1760^2 214, 121 and 129 (164), 4560 x 160 124, 57 and 45
+// (82); 3D 1560 x 160 x 160 1208, 761 and 937 (1342), 3060 x 90 x 90 1267, 671 and 609 (864).
+constexpr int kLongColumn = 1200;
+
 template <int MODE>
 void launch_line(const PsLap* P, const FftDev& d, int axis, int lpb, int others, hipStream_t s)
 {
@@ -585,7 +592,7 @@ void launch_line(const PsLap* P, const FftDev& d, int axis, int lpb, int others,
     if (lpb == 16) hipLaunchKernelGGL((k_ps_line<MODE, 16, 256>), grid, dim3(256), lds, s, d, g, P->tmp, axis, P->lapl);
     else if (lpb == 8) hipLaunchKernelGGL((k_ps_line<MODE, 8, 128>), grid, dim3(128), lds, s, d, g, P->tmp, axis, P->lapl);
     else if (lpb == 4) hipLaunchKernelGGL((k_ps_line<MODE, 4, 64>), grid, dim3(64), lds, s, d, g, P->tmp, axis, P->lapl);
-    else hipLaunchKernelGGL((k_ps_line<MODE, 1, 64>), grid, dim3(64), lds, s, d, g, P->tmp, axis, P->lapl);
+    else hipLaunchKernelGGL((k_ps_line<MODE, 1, 256>), grid, dim3(256), lds, s, d, g, P->tmp, axis, P->lapl);
 }
 
 template <bool D3>
@@ -601,14 +608,16 @@ void launch_z(const PsLap* P, const PsStep& a, int inv, int fwd, hipStream_t s, 
         hipExtLaunchKernelGGL((k_ps_z<D3, 8, 128>), grid, dim3(128), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
     else if (lpb == 4)
         hipExtLaunchKernelGGL((k_ps_z<D3, 4, 64>), grid, dim3(64), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
+    else if (g.h > kLongColumn)
+        hipExtLaunchKernelGGL((k_ps_z<D3, 1, 512>), grid, dim3(512), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
     else
-        hipExtLaunchKernelGGL((k_ps_z<D3, 1, 64>), grid, dim3(64), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
+        hipExtLaunchKernelGGL((k_ps_z<D3, 1, 256>), grid, dim3(256), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
 }
 
 // Lines per block: 16 (128 B segments) where at least two blocks per CU remain and the buffers
 // leave room for several blocks per CU, else fewer.  Measured, 16 against 8 and 4 lines along x and
 // y and along z: 144^3 (141^3 updated) 59, 76 and 100 us a step, 120^3 40, 53 and 67 us; one line
-// against four on the 2D 192 x 240 grid 17.9 against 20.5 (x) and 22.7 us (z).
+// (64 threads) against four on the 2D 192 x 240 grid 17.9 against 20.5 (x) and 22.7 us (z).
 int lines_per_block(long long lines, int others, size_t (*lds)(int, int), int n)
 {
     for (int l : {16, 8, 4})
@@ -692,9 +701,8 @@ PsLap* ps_create(int n1, int n2, int n3, int ldz, long long ldxy, float dz, floa
     P->lz = lines_per_block(n2, n3, z_lds, g.h);
     P->lx = lines_per_block(nk, n3, n3 > 1 ? +one : +both, n2);
     P->ly = lines_per_block(nk, n2, both, n3);
-    // A line that has a wave of its own (small grids, where a launch is one chain of latencies) runs
-    // one level per pass: 60 threads of a 240-point line share each pass, 16 would share a pair of
-    // levels (2D 181 x 227 step: 17.9 against 20.6 us).
+    // A line that has a block of its own runs one level per pass: 60 threads of a 240-point line share
+    // each pass, 16 would share a pair of levels (2D 181 x 227 step, 64 threads: 17.9 against 20.6 us).
     if (!rc) rc = make_dev(P, g.h, P->lz > 1, P->z, err);
     if (!rc) rc = make_dev(P, n2, P->lx > 1, P->x, err);
     if (!rc && n3 > 1) rc = make_dev(P, n3, P->ly > 1, P->y, err);

@@ -138,3 +138,27 @@ def test_spectral_extents_refused(shape, what):
         assert what in L.pw_last_error(ctx).decode()
     finally:
         L.pw_afd_destroy(p)
+
+
+@pytest.mark.parametrize("shape", [(4490, 5), (2990, 7), (2420, 6), (2390, 6), (1300, 9), (6, 1790), (4490, 3, 4), (84, 85, 180)])
+def test_aps_long_lines_vs_oracle(shape):
+    # z columns of 512- and 256-thread blocks, up to 99 KB of LDS (2250 pairs; 66 KB at 1500) and more
+    # cells than a block loads at once, an x line of 1800 points, and 190-point y lines whose operator
+    # values take a second round of loads; same operations in the same order as the oracle's, so equal
+    rng = np.random.default_rng(sum(shape))
+    nt, dt, nbt, d2, d3 = 4, 0.0005, 5, (9.0, 10.0), (12.0, 10.0, 11.0)
+    vel = (1700 + 900 * rng.random(shape)).astype(np.float32)
+    wav = rng.standard_normal((1, nt)).astype(np.float32)
+    s = [n // 2 for n in shape[1:]] + [min(1, shape[0] - 1)]
+    if len(shape) == 2:
+        d, snaps, _ = O.afd2d(vel, nt, dt, d2[1], d2[0], nbt, 0.03, s[:1], s[1:], wav, jsnap=3, ps=True)
+    else:
+        d, snaps, _ = O.afd3d(vel, nt, dt, d3[1], d3[2], d3[0], nbt, 0.03, s[:1], s[1:2], s[2:], wav, jsnap=3, ps=True)
+    p = AfdPlan(vel, d2 if len(shape) == 2 else d3, nt, dt, nbt, 0.03, 3, spectral=True)
+    p.set_sources(np.array(s + [25, 0.002, 1.0], np.float32), 1, wavelet=wav)
+    p.run()
+    out = p.output()
+    n = nt * int(np.prod(shape[1:]))
+    assert np.array_equal(out[:n].reshape((nt,) + shape[1:], order="F"), d.T)
+    w = out[n:].reshape(shape + (-1,), order="F")
+    assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
