@@ -383,3 +383,26 @@ def test_afd2d_multi_step_launches_vs_oracle(shape, nbt, nt, tri):
         w = out[nt * nx:].reshape(nz, nx, -1, order="F")
         assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
     p.close()
+
+
+@pytest.mark.parametrize("shape,ns", [((40, 37), 63), ((40, 37), 64), ((40, 37), 65), ((70, 130), 200), ((640, 500), 300)])
+def test_afd2d_many_sources_vs_oracle(shape, ns):
+    # source counts around the 64 a strip holds in registers, several sources on one cell, sources whose
+    # stencils cross strips and tiles: added in source order as the oracle does, so equal
+    rng = np.random.default_rng(ns + shape[0])
+    nz, nx = shape
+    nt, dt, dz, dx, nbt = 11, 0.001, 9.0, 11.0, 6
+    vel = (1500 + 1500 * rng.random(shape)).astype(np.float32)
+    sx, sz = rng.integers(0, nx, ns), rng.integers(0, nz, ns)
+    sx[-3:], sz[-3:] = sx[0], sz[0]
+    wav = rng.standard_normal((ns, nt)).astype(np.float32)
+    d, snaps, _ = O.afd2d(vel, nt, dt, dx, dz, nbt, 0.02, list(sx), list(sz), wav, jsnap=10)
+    p = AfdPlan(vel, (dz, dx), nt, dt, nbt, 0.02, 10)
+    pack = np.concatenate([sx, sz, np.full(ns, 20), np.full(ns, 0.002), np.ones(ns)]).astype(np.float32)
+    p.set_sources(pack, ns, wavelet=wav)
+    p.run()
+    out = p.output()
+    assert np.array_equal(out[:nt * nx].reshape(nt, nx, order="F"), d.T)
+    w = out[nt * nx:].reshape(nz, nx, -1, order="F")
+    assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
+    p.close()
