@@ -2039,11 +2039,20 @@ int pw_afd_final_field(pw_afd* p, float* out, long long out_len)
     if (!p->final_field) PW_FAIL(ctx, PW_ERR_STATE, "final_field: nothing has run");
     hipStream_t s = ctx->s();
     if (int rc = pw::check_finite(ctx, p->final_field, p->field_elems, 4, "afd: final wavefield")) return rc;
+    // gathered in the transpose scratch (nt samples a trace) where the model's columns fit it
+    float* own = nullptr;
+    if (g.nz1 > p->nt) {
+        PW_HIP(ctx, hipSetDevice(ctx->device));
+        PW_HIP(ctx, hipMalloc(&own, n * 4));
+    }
+    float* d = own ? own : p->d_tmp;
     dim3 grid(pw::ceil_div(g.nz1, 256), g.nx1, g.ny1);
-    hipLaunchKernelGGL(k_interior, grid, dim3(256), 0, s, g, p->final_field, p->d_tmp);
-    PW_HIP(ctx, hipGetLastError());
-    PW_HIP(ctx, hipMemcpyAsync(out, p->d_tmp, n * 4, hipMemcpyDeviceToHost, s));
-    PW_HIP(ctx, hipStreamSynchronize(s));
+    hipLaunchKernelGGL(k_interior, grid, dim3(256), 0, s, g, p->final_field, d);
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(out, d, n * 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    if (own) hipFree(own);
+    if (e != hipSuccess) PW_FAIL(ctx, PW_ERR_HIP, std::string("final_field: ") + hipGetErrorString(e));
     return PW_OK;
 }
 

@@ -406,3 +406,17 @@ def test_afd2d_many_sources_vs_oracle(shape, ns):
     w = out[nt * nx:].reshape(nz, nx, -1, order="F")
     assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
     p.close()
+
+
+@pytest.mark.parametrize("shape,nt", [((200, 31), 3), ((31, 40), 31), ((300, 12, 7), 2)])
+def test_final_field_of_runs_shorter_than_the_columns(shape, nt):
+    # fewer time steps than samples along z: the field has more values than the run has trace samples
+    rng = np.random.default_rng(nt)
+    vel = (1500 + 1500 * rng.random(shape)).astype(np.float32)
+    p = AfdPlan(vel, (10.0,) * len(shape), nt, 0.001, 5, 0.01, nt - 1)
+    cells = [n // 2 for n in shape[1:]] + [shape[0] // 2]
+    p.set_sources(np.array(cells + [10, 0.002, 1], np.float32), 1, wavelet=rng.standard_normal((1, nt)).astype(np.float32))
+    p.run()
+    last = p.output()[nt * int(np.prod(shape[1:])):].reshape(shape + (-1,), order="F")[..., -1]
+    assert np.array_equal(p.final_field(), last) and last.any()
+    p.close()
