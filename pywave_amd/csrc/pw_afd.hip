@@ -876,10 +876,10 @@ __global__ __launch_bounds__(64 * WAVES) void k_afd3d_2step(Geo g, Step2 a, int 
 }
 
 // ---------------------------------------------------------------- 2D: K steps per launch
-template <int K, int S, int W>
+template <int K, int S, int W, bool MANY>
 __global__ __launch_bounds__(64 * W) void k_afd2d_multi(pw2d::Steps a)
 {
-    pw2d::advance<K, S, W>(a, blockIdx.x, blockIdx.y);
+    pw2d::advance<K, S, W, MANY>(a, blockIdx.x, blockIdx.y);
 }
 
 // ---------------------------------------------------------------- 2D: one cell per lane
@@ -1528,7 +1528,8 @@ int afd_launch_multi(pw_afd* p, int shape, const pw2d::Steps& a, hipEvent_t e0, 
         static_assert(kShapes2[I].k == K && kShapes2[I].owned_z == T::owned_z &&                               \
                       kShapes2[I].owned_x == T::owned_x, "launch shape");                                      \
         const dim3 grid(pw::ceil_div(g.nz, T::owned_z), pw::ceil_div(g.nx, T::owned_x));                       \
-        hipExtLaunchKernelGGL((k_afd2d_multi<K, S, W>), grid, dim3(64 * W), 0, s, e0, e1, 0, a);               \
+        if (a.ns > 1) hipExtLaunchKernelGGL((k_afd2d_multi<K, S, W, true>), grid, dim3(64 * W), 0, s, e0, e1, 0, a); \
+        else hipExtLaunchKernelGGL((k_afd2d_multi<K, S, W, false>), grid, dim3(64 * W), 0, s, e0, e1, 0, a);   \
         break;                                                                                                 \
     }
     switch (shape) {

@@ -42,7 +42,12 @@ struct Tile {
     static constexpr int halo = 2 * K, owned_z = 64 - 4 * K, cols = S * W, owned_x = cols - 4 * K;
 };
 
-template <int K, int S, int W>
+// MANY: how a strip finds its sources.  With MANY strips look at the sources 64 at a time, one per
+// lane; without, every strip of a tile that some source reaches goes through all of them, read as
+// scalars.  The latter is faster for one source (161^2 cells, near the receivers' row, 1.34 against
+// 1.37 us a step); with two it is slower (263 x 457 cells 1.65 against 1.46), with 100 and 1000 it takes
+// 24.5 and 238 us against 2.0 and 6.5.
+template <int K, int S, int W, bool MANY>
 __device__ __forceinline__ void advance(const Steps& a, int tz, int tx)
 {
     using T = Tile<K, S, W>;
@@ -55,10 +60,8 @@ __device__ __forceinline__ void advance(const Steps& a, int tz, int tx)
     const int L = a.ldz;
     const bool zact = z >= 0 && z < a.nz;
     const bool zin = zact && z >= 2 && z < a.nz2 - 2;
-    // Sources i0 .. i0 + 63, one per lane: their row, kFar where the stencil misses the strip.  The first
-    // 64, loaded ahead of the fields, stay in registers over the launch.  (Strips that each looped over
-    // every source of the run took 24.5 and 238 us a step for 100 and 1000 sources on 263 x 457 cells,
-    // single steps, one cell per lane, 13.8 and 107; this takes 2.1 and 6.9.)
+    // MANY: sources i0 .. i0 + 63, one per lane: their row, kFar where the stencil misses the strip.  The
+    // first 64, loaded ahead of the fields, stay in registers over the launch.
     constexpr int kFar = -1;  // no source's: their stencils lie inside the grid
     auto near = [&](int i0, int& sx) -> int {
         const int i = i0 + lane;
@@ -68,7 +71,7 @@ __device__ __forceinline__ void advance(const Steps& a, int tz, int tx)
         return sz >= z0 - 1 && sz <= z0 + 64 && sx >= xs - 1 && sx <= xs + S ? sz : kFar;
     };
     int sx0 = 0;
-    const int sz0 = near(0, sx0);
+    const int sz0 = MANY ? near(0, sx0) : kFar;
     float u[S], p[S], vc[S], fx[S];
     unsigned lapmask[S];
     float fzz = 1.f;
@@ -95,8 +98,14 @@ __device__ __forceinline__ void advance(const Steps& a, int tz, int tx)
         // zero on the Laplacian's rim and outside the updated domain, whose cells so stay zero
         lapmask[s] = zin && xact && x >= 2 && x < a.nx2 - 2 ? ~0u : 0u;
     }
-    bool hit = __ballot(sz0 != kFar) != 0;  // some source's stencil reaches the strip
-    for (int i0 = 64, sx; i0 < a.ns; i0 += 64) hit |= __ballot(near(i0, sx) != kFar) != 0;
+    bool hit = false;  // some source's stencil reaches the strip (without MANY: the tile)
+    if constexpr (MANY) {
+        hit = __ballot(sz0 != kFar) != 0;
+        for (int i0 = 64, sx; i0 < a.ns; i0 += 64) hit |= __ballot(near(i0, sx) != kFar) != 0;
+    } else {
+        for (int s = 0; s < a.ns; ++s)
+            hit |= a.src[3 * s] >= z0 - 1 && a.src[3 * s] <= z0 + 64 && a.src[3 * s + 1] >= x0 - 1 && a.src[3 * s + 1] <= x0 + NX;
+    }
     // the receiver row's lane, if the tile holds it; and if the tile owns it
     const int rlane = a.nb - z0;
     const bool rtile = rlane >= 0 && rlane < 64, rowned = rlane >= H && rlane < 64 - H;
@@ -152,16 +161,30 @@ __device__ __forceinline__ void advance(const Steps& a, int tz, int tx)
             c = c + lap * vc[s];
             nu[s] = c;
         }
-        if (hit) {
-            for (int i0 = 0, sz = sz0, sx = sx0; i0 < a.ns; i0 += 64) {  // in source order
-                if (i0) sz = near(i0, sx);
-                for (unsigned long long m = __ballot(sz != kFar); m; m &= m - 1) {
-                    const int i = __builtin_ctzll(m);
-                    const int dz = abs(z - __builtin_amdgcn_readlane(sz, i)), gx = __builtin_amdgcn_readlane(sx, i);
-                    const float wv = a.wav[(size_t)(i0 + i) * a.nt + t];
+        if (hit) {  // in source order
+            if constexpr (MANY) {
+                for (int i0 = 0, sz = sz0, sx = sx0; i0 < a.ns; i0 += 64) {
+                    if (i0) sz = near(i0, sx);
+                    for (unsigned long long m = __ballot(sz != kFar); m; m &= m - 1) {
+                        const int i = __builtin_ctzll(m);
+                        const int dz = abs(z - __builtin_amdgcn_readlane(sz, i)), gx = __builtin_amdgcn_readlane(sx, i);
+                        const float wv = a.wav[(size_t)(i0 + i) * a.nt + t];
+#pragma unroll
+                        for (int s = 0; s < S; ++s) {
+                            const int dx = abs(xs + s - gx);
+                            if (dx > 1) continue;
+                            asm volatile("");  // a branch, not the quotients of every column and a select
+                            if (dz <= 1) nu[s] = nu[s] + (vc[s] * wv) / (float)(dz + dx + 1);
+                        }
+                    }
+                }
+            } else {
+                for (int i = 0; i < a.ns; ++i) {
+                    const int dz = abs(z - a.src[3 * i]);
+                    const float wv = a.wav[(size_t)i * a.nt + t];
 #pragma unroll
                     for (int s = 0; s < S; ++s) {
-                        const int dx = abs(xs + s - gx);
+                        const int dx = abs(xs + s - a.src[3 * i + 1]);
                         if (dz <= 1 && dx <= 1) nu[s] = nu[s] + (vc[s] * wv) / (float)(dz + dx + 1);
                     }
                 }
