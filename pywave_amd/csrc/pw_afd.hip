@@ -1332,7 +1332,7 @@ struct pw_afd {
     float* d_snap = nullptr;  // [ntsnap][ny1][nx1][nz1]
     float* d_tmp = nullptr;   // transpose scratch (nrec*nt)
     float* raw[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // behind d_a, d_b, d_vv, d_c, d_d (guarded)
-    float* d_c = nullptr;  // the two extra fields of the two-step kernels (allocated on first use)
+    float* d_c = nullptr;  // the two extra fields of the two-step 3D and the multi-step 2D kernels (null: none yet)
     float* d_d = nullptr;
     size_t raw_elems = 0, guard_lo = 0;
     float* d_fz1 = nullptr;  // single damping factor per index (lean kernels)
@@ -1425,6 +1425,13 @@ int afd_launch_step(pw_afd* p, const Step& a, hipEvent_t e0 = nullptr, hipEvent_
     pw_ctx* ctx = p->ctx;
     hipStream_t s = ctx->s();
     const Geo& g = p->g;
+    if (p->ndim == 2) {
+        constexpr int W = 4;
+        dim3 grid(pw::ceil_div(g.nz, 64), pw::ceil_div(g.nx, W));
+        hipExtLaunchKernelGGL(k_afd2d<W>, grid, dim3(64 * W), 0, s, e0, e1, 0, g, a);
+        PW_HIP(ctx, hipGetLastError());
+        return PW_OK;
+    }
     const int vi = p->variant >= 0 ? p->variant : default_variant(p);
     const Variant3 v = kVariants3[vi];
     if (!variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "3D kernel variant not applicable to this grid");
@@ -1592,6 +1599,25 @@ void afd_free(pw_afd* p)
     ps_destroy(p->ps);
 }
 
+constexpr size_t kOneBlockBytes = (size_t)16 << 20;  // 2D fields up to this size share one allocation of five
+
+// The second pair of fields of the 2D multi-step launches; without it a run takes one step per
+// launch.  Spectral plans have no use for it.
+int second_pair(pw_afd* p)
+{
+    if (p->ndim != 2 || p->ps || p->d_c) return PW_OK;
+    PW_HIP(p->ctx, hipSetDevice(p->ctx->device));
+    if (hipMalloc(&p->raw[3], 2 * p->raw_elems * 4) != hipSuccess) {
+        (void)hipGetLastError();  // must not surface as a later launch error
+        p->raw[3] = nullptr;
+        return PW_OK;
+    }
+    p->d_c = p->raw[3];
+    p->d_d = p->d_c + p->raw_elems;
+    PW_HIP(p->ctx, hipMemsetAsync(p->d_c, 0, 2 * p->raw_elems * 4, p->ctx->s()));
+    return PW_OK;
+}
+
 int afd_check(pw_afd* p) { return p && p->ctx ? PW_OK : PW_ERR_ARG; }
 
 }  // namespace
@@ -1695,9 +1721,10 @@ pw_afd* pw_afd_create(pw_ctx* ctx, int ndim, int nz, int nx, int ny, float dz, f
     p->chunk_ok = lean && max_chunk_planes(g) >= 1;
 
     const size_t nrec = (size_t)g.nx1 * g.ny1;
-    // 3D: three fields (two more when a two-step kernel first runs); 2D: the five fields of the
-    // multi-step launches in one allocation, as its cost counts in a one-shot call on a small grid
-    const size_t nfield = ndim == 2 ? 5 : 1;
+    // Three fields, and two more for the multi-step 2D kernels (with the velocity) or the two-step 3D
+    // ones (when one first runs).  In 2D they are one allocation, the second pair included on small
+    // grids: another allocation and its release add 12 us to a one-shot call of 1.6 ms on 161^2 cells.
+    const size_t nfield = ndim != 2 ? 1 : p->raw_elems * 4 <= kOneBlockBytes ? 5 : 3;
     bool ok = hipMalloc(&p->raw[0], nfield * p->raw_elems * 4) == hipSuccess &&
               (ndim == 2 || (hipMalloc(&p->raw[1], p->raw_elems * 4) == hipSuccess &&
                              hipMalloc(&p->raw[2], p->raw_elems * 4) == hipSuccess)) &&
@@ -1714,8 +1741,10 @@ pw_afd* pw_afd_create(pw_ctx* ctx, int ndim, int nz, int nx, int ny, float dz, f
             p->d_a = p->raw[0];
             p->d_b = p->d_a + p->raw_elems;
             p->d_vv = p->d_b + p->raw_elems;
-            p->d_c = p->d_vv + p->raw_elems;
-            p->d_d = p->d_c + p->raw_elems;
+            if (nfield == 5) {
+                p->d_c = p->d_vv + p->raw_elems;
+                p->d_d = p->d_c + p->raw_elems;
+            }
         } else {
             p->d_a = p->raw[0] + p->guard_lo;
             p->d_b = p->raw[1] + p->guard_lo;
@@ -1734,7 +1763,7 @@ pw_afd* pw_afd_create(pw_ctx* ctx, int ndim, int nz, int nx, int ny, float dz, f
     ok = hipMemcpyAsync(p->d_fz, fz.data(), fz.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
          hipMemcpyAsync(p->d_fx, fx.data(), fx.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
          hipMemcpyAsync(p->d_fy, fy.data(), fy.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
-         hipMemsetAsync(p->d_vv - p->guard_lo, 0, (ndim == 2 ? 3 : 1) * p->raw_elems * 4, s) == hipSuccess &&
+         hipMemsetAsync(p->d_vv - p->guard_lo, 0, (nfield == 5 ? 3 : 1) * p->raw_elems * 4, s) == hipSuccess &&
          (!lean || (hipMemcpyAsync(p->d_fz1, fz1.data(), fz1.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
                     hipMemcpyAsync(p->d_fx1, fx1.data(), fx1.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess &&
                     hipMemcpyAsync(p->d_fy1, fy1.data(), fy1.size() * 4, hipMemcpyHostToDevice, s) == hipSuccess)) &&
@@ -1762,6 +1791,7 @@ int pw_afd_set_velocity(pw_afd* p, const float* vel)
     if (afd_check(p) || !vel) return PW_ERR_ARG;
     pw_ctx* ctx = p->ctx;
     const Geo& g = p->g;
+    if (int rc = second_pair(p)) return rc;
     size_t n = (size_t)g.nz1 * g.nx1 * g.ny1;
     float* d_vel = nullptr;
     PW_HIP(ctx, hipMalloc(&d_vel, n * 4));
@@ -1856,7 +1886,7 @@ static int afd_enqueue(pw_afd* p, int tri, hipEvent_t* evs, int nsteps = 0, bool
     hipStream_t s = ctx->s();
     const int vi = p->ndim == 3 && !p->ps ? (p->variant >= 0 ? p->variant : default_variant(p)) : -1;
     const bool two = vi >= 0 && kVariants3[vi].lean == 5;
-    const bool multi = p->ndim == 2 && !p->ps;
+    const bool multi = p->ndim == 2 && !p->ps && p->d_c;
     const int shape2 = multi ? shape2_of(g) : 0;
     if (two && !variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "two-step 3D kernel not applicable to this grid");
     if (two && !p->d_c) {
@@ -2130,7 +2160,7 @@ int pw_afd_set_spectral(pw_afd* p, int on)
     pw_ctx* ctx = p->ctx;
     if (!on) {
         ps_destroy(p->ps);
-        p->ps = nullptr;
+        p->ps = nullptr;  // without a second pair of fields until the velocity is set again
         return PW_OK;
     }
     if (p->ps) return PW_OK;

@@ -420,3 +420,39 @@ def test_final_field_of_runs_shorter_than_the_columns(shape, nt):
     last = p.output()[nt * int(np.prod(shape[1:])):].reshape(shape + (-1,), order="F")[..., -1]
     assert np.array_equal(p.final_field(), last) and last.any()
     p.close()
+
+
+def test_spectral_2d_plans_hold_no_second_pair():
+    # three fields, the half spectrum and its operator: 4.5 padded fields, 6.5 with the pair that
+    # multi-step launches need
+    torch = pytest.importorskip("torch")
+    vel = np.full((4000, 1700), 2000, np.float32)
+    for _ in range(2):  # the first plan also loads kernels
+        free = torch.cuda.mem_get_info()[0]
+        p = AfdPlan(vel, (10.0, 10.0), 2, 0.001, 30, 0.01, 0, spectral=True)
+        used = free - torch.cuda.mem_get_info()[0]
+        p.close()
+    assert used < 5.5 * 4 * 4096 * 1800
+
+
+@pytest.mark.parametrize("tri", [False, True])
+def test_2d_plan_without_second_pair_takes_single_steps(tri):
+    # what a plan does that found no room for the pair: here one that was spectral when its velocity
+    # was set, on a grid whose pair has an allocation of its own; the same traces and snapshots as in
+    # multi-step launches
+    nt, shape = 7, (2500, 1730)
+    rng = np.random.default_rng(2)
+    vel = (1500 + 1500 * rng.random(shape)).astype(np.float32)
+    out = []
+    for spectral in (False, True):
+        p = AfdPlan(vel, (10.0, 10.0), nt, 0.001, 30, 0.01, 3, spectral=spectral)
+        if spectral:
+            assert p._L.pw_afd_set_spectral(p._p, 0) == 0
+        p.set_sources(np.array([950, 951, 1090, 1095, 10, 10, 0.002, 0.002, 1, 1], np.float32), 2,
+                      wavelet=np.random.default_rng(5).standard_normal((2, nt)).astype(np.float32))
+        p.set_tri_data(np.random.default_rng(6).standard_normal((nt, shape[1])).astype(np.float32))
+        p.run(tri=tri)
+        out.append((p.output(), p.final_field()))
+        p.close()
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][0].any()
+    assert np.array_equal(out[0][1], out[1][1])
