@@ -2101,8 +2101,14 @@ int pw_afd_autotune(pw_afd* p, int steps, int* variant_out, int* chunk_out)
         return PW_OK;
     }
     const auto key = std::make_tuple(g.nz2, g.nx2, g.ny2);
-    auto it = ctx->tuned.find(key);
-    if (it == ctx->tuned.end()) {
+    std::pair<int, int> choice(default_variant(p), 0);
+    bool known = false;
+    {
+        std::lock_guard<std::mutex> lk(ctx->choice_mu);
+        auto it = ctx->tuned.find(key);
+        if ((known = it != ctx->tuned.end())) choice = it->second;
+    }
+    if (!known) {
         if (!p->have_vel) PW_FAIL(ctx, PW_ERR_STATE, "autotune: velocity not set");
         hipStream_t s = ctx->s();
         hipEvent_t e0, e1;
@@ -2110,7 +2116,6 @@ int pw_afd_autotune(pw_afd* p, int steps, int* variant_out, int* chunk_out)
         PW_HIP(ctx, hipEventCreate(&e1));
         const int chunks[] = {0, 4, 6, 8, 12, 16, 24, 32, 48};
         float best = 1e30f;
-        std::pair<int, int> choice(default_variant(p), 0);
         const int saved_v = p->variant, saved_c = p->ny_chunk;
         const int nst = std::max(2, steps + (steps & 1));  // even: two-step kernels run whole launches
         const int mode = p->have_src ? 0 : 1;                 // time the plan's own kind of run
@@ -2144,10 +2149,11 @@ int pw_afd_autotune(pw_afd* p, int steps, int* variant_out, int* chunk_out)
         p->ny_chunk = saved_c;
         hipEventDestroy(e0);
         hipEventDestroy(e1);
-        it = ctx->tuned.emplace(key, choice).first;
+        std::lock_guard<std::mutex> lk(ctx->choice_mu);
+        ctx->tuned[key] = choice;
     }
-    p->variant = it->second.first;
-    p->ny_chunk = it->second.second;
+    p->variant = choice.first;
+    p->ny_chunk = choice.second;
     if (variant_out) *variant_out = p->variant;
     if (chunk_out) *chunk_out = p->ny_chunk;
     return PW_OK;
@@ -2578,12 +2584,12 @@ int tri_ensure_tuned(pw_tri* p)
     const Geo& g = p->g;
     const int gk = std::min(kTriPassGroups, p->G);
     const std::vector<long long> key = {4, gk, g.nz, g.nx, g.ny};
-    auto hit = p->ctx->tuned2d.find(key);
-    if (hit != p->ctx->tuned2d.end()) {
-        p->tri_w = hit->second.first[0];
-        p->tri_nyc = hit->second.first[1];
-        p->tri_nt = hit->second.first[2];
-        p->tune_log = hit->second.second;
+    pw_ctx::Choice known;
+    if (p->ctx->find_choice(key, &known)) {
+        p->tri_w = known.first[0];
+        p->tri_nyc = known.first[1];
+        p->tri_nt = known.first[2];
+        p->tune_log = known.second;
         p->tuned = true;
         return PW_OK;
     }
@@ -2594,7 +2600,7 @@ int tri_ensure_tuned(pw_tri* p)
         case 3: rc = tri_tune<3>(p); break;
         default: rc = tri_tune<4>(p); break;
     }
-    if (!rc) p->ctx->tuned2d[key] = {{p->tri_w, p->tri_nyc, p->tri_nt}, p->tune_log};
+    if (!rc) p->ctx->keep_choice(key, {{p->tri_w, p->tri_nyc, p->tri_nt}, p->tune_log});
     return rc;
 }
 

@@ -378,11 +378,11 @@ std::vector<long long> tune_key(const pw_batch* p)
 int tune_width(pw_batch* p)
 {
     const std::vector<long long> key = tune_key(p);
-    auto hit = p->ctx->tuned2d.find(key);
-    if (hit != p->ctx->tuned2d.end()) {
-        p->tune_log = hit->second.second;
+    pw_ctx::Choice known;
+    if (p->ctx->find_choice(key, &known)) {
+        p->tune_log = known.second;
         p->tuned = true;
-        return apply_layout(p, hit->second.first[0]);
+        return apply_layout(p, known.first[0]);
     }
     hipStream_t st = p->ctx->s();
     p->tune_log.clear();
@@ -423,7 +423,7 @@ int tune_width(pw_batch* p)
     int rc = apply_layout(p, best);
     if (rc) return rc;
     p->tuned = true;
-    p->ctx->tuned2d[key] = {{best}, p->tune_log};
+    p->ctx->keep_choice(key, {{best}, p->tune_log});
     return PW_OK;
 }
 

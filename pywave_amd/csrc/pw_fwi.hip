@@ -2897,9 +2897,9 @@ int ensure_widths(pw_fwi* p)
 {
     if (p->widths_tuned) return PW_OK;
     const std::vector<long long> key = tune_key(p);
-    auto hit = p->ctx->tuned2d.find(key);
-    if (hit != p->ctx->tuned2d.end()) {
-        const std::vector<int>& w = hit->second.first;
+    pw_ctx::Choice known;
+    if (p->ctx->find_choice(key, &known)) {
+        const std::vector<int>& w = known.first;
         p->w_fwd = w[0]; p->w_fwdv = w[1]; p->w_exact = w[2]; p->w_ref = w[3]; p->w_refv = w[4];
         p->w_fwd2 = w[5]; p->w_adj2 = w[6]; p->w_fwdt = w[7];
         const long long fld = p->nslot * p->fs;
@@ -2909,15 +2909,14 @@ int ensure_widths(pw_fwi* p)
         if (!rc && p->w_adj2 && !p->A2) rc = dmalloc(p, &p->A2, fld * 4);
         if (!rc && p->w_adj2 && !p->B2) rc = dmalloc(p, &p->B2, fld * 4);
         if (rc) return rc;
-        p->tune_log = hit->second.second;  // the sweep of the earlier plan that chose them
+        p->tune_log = known.second;  // the sweep of the earlier plan that chose them
         p->widths_tuned = true;
         return PW_OK;
     }
     int rc = p->prec == 4 ? tune_widths<float>(p) : tune_widths<double>(p);
     if (!rc)
-        p->ctx->tuned2d[key] = {{p->w_fwd, p->w_fwdv, p->w_exact, p->w_ref, p->w_refv, p->w_fwd2, p->w_adj2,
-                                 p->w_fwdt},
-                                p->tune_log};
+        p->ctx->keep_choice(key, {{p->w_fwd, p->w_fwdv, p->w_exact, p->w_ref, p->w_refv, p->w_fwd2, p->w_adj2, p->w_fwdt},
+                                  p->tune_log});
     return rc;
 }
 

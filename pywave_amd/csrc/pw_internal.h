@@ -6,6 +6,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <map>
+#include <mutex>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -18,12 +19,29 @@ struct pw_ctx {
     hipStream_t ext_stream = nullptr;  // caller stream (may be the null stream) when use_ext
     bool use_ext = false;
     std::string err;
-    // autotuned 3D step choice per padded grid shape: (nz2, nx2, ny2) -> (variant, y chunk)
+    // Launch choices that a plan's timing sweep made, shared by the context's plans; the one-shot calls
+    // of several threads run on one context, so they are read and written under the lock.
+    std::mutex choice_mu;
+    // 3D step kernel (pw_afd_autotune) per padded grid shape: (nz2, nx2, ny2) -> (variant, y chunk)
     std::map<std::tuple<int, int, int>, std::pair<int, int>> tuned;
-    // autotuned 2D tile widths per workload key (kind, padded shapes, shots per launch and what
-    // else decides which tiles run the general loop) -> the widths a plan's timing sweep chose,
-    // then that sweep's log (kernel, width, ms per launch)
-    std::map<std::vector<long long>, std::pair<std::vector<int>, std::vector<float>>> tuned2d;
+    // per workload key -- the kind (1 batched 2D, 2 FWI, 3 LS-TRI, 4 time-reversal image), grid, shots or
+    // groups per launch and what else decides the outcome -- the choice (tile widths, steps per launch,
+    // rows and y chunk) and its sweep's log (kernel, shape, ms per launch)
+    using Choice = std::pair<std::vector<int>, std::vector<float>>;
+    std::map<std::vector<long long>, Choice> choices;
+    bool find_choice(const std::vector<long long>& key, Choice* out)
+    {
+        std::lock_guard<std::mutex> lk(choice_mu);
+        auto hit = choices.find(key);
+        if (hit == choices.end()) return false;
+        *out = hit->second;
+        return true;
+    }
+    void keep_choice(const std::vector<long long>& key, Choice c)
+    {
+        std::lock_guard<std::mutex> lk(choice_mu);
+        choices[key] = std::move(c);
+    }
     unsigned* d_count = nullptr;  // device counter of pw::count_nonfinite (allocated on first use)
     hipStream_t s() const { return use_ext ? ext_stream : stream; }
 };

@@ -919,10 +919,10 @@ int select_launch(pw_lstri* p, int nslot)
     auto own = p->choice.find(nslot);
     if (own == p->choice.end()) {
         const std::vector<long long> key = {3, p->g.pz, p->g.px, p->g.nb, p->g.depth, p->nz, p->nx, p->nt, nslot};
-        auto hit = p->ctx->tuned2d.find(key);
-        if (hit != p->ctx->tuned2d.end()) {
-            p->tune_log = hit->second.second;
-            own = p->choice.emplace(nslot, hit->second.first).first;
+        pw_ctx::Choice known;
+        if (p->ctx->find_choice(key, &known)) {
+            p->tune_log = known.second;
+            own = p->choice.emplace(nslot, known.first).first;
         } else {
             int rc = ensure_fields(p, nslot);
             if (!rc) rc = ensure_batch(p, nslot);
@@ -974,7 +974,7 @@ int select_launch(pw_lstri* p, int nslot)
                 }
             }
             own = p->choice.emplace(nslot, std::vector<int>{wbest, sbest, obest}).first;
-            p->ctx->tuned2d[key] = {own->second, p->tune_log};
+            p->ctx->keep_choice(key, {own->second, p->tune_log});
         }
     }
     p->xct = p->xct_forced ? p->xct_forced : own->second[0];

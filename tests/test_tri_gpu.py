@@ -137,3 +137,21 @@ def test_every_launch_shape_gives_the_same_image():
         assert np.array_equal(img, ref), (rows, chunk, nt_)
     with pytest.raises(ValueError):
         pywave_amd.tri3d_image(vel, dat, groups, launch=(5, 4), **kw)
+
+
+def test_images_of_several_threads_share_one_context():
+    # the one-shot calls run on the device's shared context, whose table of launch choices every first
+    # image of a grid reads and extends: images formed by four threads equal those formed one by one
+    from concurrent.futures import ThreadPoolExecutor
+    rng = np.random.default_rng(12)
+    cases = []
+    for k in range(12):
+        nz, nx, ny = (int(n) for n in rng.integers(9, 30, 3))
+        vel = (1500 + 1500 * rng.random((nz, nx, ny))).astype(np.float32)
+        dat = rng.standard_normal((15, nx, ny)).astype(np.float32)
+        kw = dict(ax=[0, 20, nx], ay=[0, 20, ny], az=[0, 20, nz], nbt=6, jsnap=2)
+        cases.append((vel, dat, [np.arange(g, nx, 1 + k % 3) for g in range(1 + k % 3)], kw))
+    with ThreadPoolExecutor(4) as pool:
+        together = list(pool.map(lambda c: pywave_amd.tri3d_image(c[0], c[1], c[2], **c[3]), cases))
+    for c, img in zip(cases, together):
+        assert np.array_equal(img, pywave_amd.tri3d_image(c[0], c[1], c[2], **c[3]))
