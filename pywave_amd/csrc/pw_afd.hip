@@ -1606,7 +1606,7 @@ constexpr size_t kOneBlockBytes = (size_t)16 << 20;  // 2D fields up to this siz
 int second_pair(pw_afd* p)
 {
     if (p->ndim != 2 || p->ps || p->d_c) return PW_OK;
-    PW_HIP(p->ctx, hipSetDevice(p->ctx->device));
+    const pw::OnDevice dev(p->ctx);
     if (hipMalloc(&p->raw[3], 2 * p->raw_elems * 4) != hipSuccess) {
         (void)hipGetLastError();  // must not surface as a later launch error
         p->raw[3] = nullptr;
@@ -1890,6 +1890,7 @@ static int afd_enqueue(pw_afd* p, int tri, hipEvent_t* evs, int nsteps = 0, bool
     const int shape2 = multi ? shape2_of(g) : 0;
     if (two && !variant_ok(p, vi)) PW_FAIL(ctx, PW_ERR_ARG, "two-step 3D kernel not applicable to this grid");
     if (two && !p->d_c) {
+        const pw::OnDevice dev(ctx);
         PW_HIP(ctx, hipMalloc(&p->raw[3], p->raw_elems * 4));
         PW_HIP(ctx, hipMalloc(&p->raw[4], p->raw_elems * 4));
         PW_HIP(ctx, hipMemsetAsync(p->raw[3], 0, p->raw_elems * 4, s));
@@ -2073,7 +2074,7 @@ int pw_afd_final_field(pw_afd* p, float* out, long long out_len)
     // gathered in the transpose scratch (nt samples a trace) where the model's columns fit it
     float* own = nullptr;
     if (g.nz1 > p->nt) {
-        PW_HIP(ctx, hipSetDevice(ctx->device));
+        const pw::OnDevice dev(ctx);
         PW_HIP(ctx, hipMalloc(&own, n * 4));
     }
     float* d = own ? own : p->d_tmp;

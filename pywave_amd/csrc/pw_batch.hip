@@ -664,7 +664,19 @@ int pw_batch2d_traces(pw_batch* p, int i, float* out, long long len)
     if (!p->d_out) {  // one shot's transposed traces, sized for the largest
         long long most = 0;
         for (const Shot& q : p->shots) most = std::max(most, (long long)q.nt * q.nx1);
-        PW_HIP(p->ctx, hipMalloc(&p->d_out, (size_t)most * 4));
+        const pw::OnDevice dev(p->ctx);
+        if (hipMalloc(&p->d_out, (size_t)most * 4) != hipSuccess) {
+            (void)hipGetLastError();  // must not surface as a later launch error
+            p->d_out = nullptr;
+        }
+    }
+    if (!p->d_out) {  // no room on the device for the run's traces in the callers' order
+        std::vector<float> t((size_t)len);
+        PW_HIP(p->ctx, hipMemcpyAsync(t.data(), p->d_rec + s.rec_off, len * 4, hipMemcpyDeviceToHost, st));
+        PW_HIP(p->ctx, hipStreamSynchronize(st));
+        for (int ix = 0; ix < s.nx1; ++ix)
+            for (int it = 0; it < s.nt; ++it) out[(size_t)ix * s.nt + it] = t[(size_t)it * s.nx1 + ix];
+        return PW_OK;
     }
     hipLaunchKernelGGL(k_traces_out, dim3(pw::ceil_div(s.nx1, 32), pw::ceil_div(s.nt, 32)), dim3(32, 8), 0, st,
                        p->d_rec + s.rec_off, p->d_out, s.nt, s.nx1);

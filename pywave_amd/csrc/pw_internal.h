@@ -84,6 +84,20 @@ int ricker(int nt, float dt, float f0, float t0, float A, float* out, std::strin
 void damping_pairs(int n2, int nb_lo, int nb_hi, const float* w_lo, const float* w_hi,
                    std::vector<float>& out2);
 
+// Makes a context's device the calling thread's until the end of a scope: buffers that a plan
+// allocates after its creation belong on its device, whichever the thread is on.
+struct OnDevice {
+    int was = -1;
+    explicit OnDevice(const pw_ctx* ctx)
+    {
+        if (hipGetDevice(&was) != hipSuccess || was == ctx->device || hipSetDevice(ctx->device) != hipSuccess) was = -1;
+    }
+    ~OnDevice()
+    {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+};
+
 template <typename T>
 inline T ceil_div(T a, T b) { return (a + b - 1) / b; }
 
