@@ -2377,6 +2377,7 @@ void fwi_free(pw_fwi* p)
 
 int dmalloc(pw_fwi* p, void** ptr, size_t bytes)
 {
+    const pw::OnDevice dev(p->ctx);
     if (hipMalloc(ptr, bytes ? bytes : 8) != hipSuccess) {
         (void)hipGetLastError();  // an out-of-memory result must not surface as a later launch error
         *ptr = nullptr;
@@ -2665,6 +2666,10 @@ int multi_fields(pw_fwi* p, bool adj)
     for (void** q : f)
         if (!*q)
             if (int rc = dmalloc(p, q, bytes)) return rc;
+    if (adj && !(p->adj_sa && p->adj_sb)) {  // a sweep that began before they were there
+        p->adj_sa = p->A2;
+        p->adj_sb = p->B2;
+    }
     return PW_OK;
 }
 
@@ -3125,7 +3130,6 @@ int adjoint_segment_multi(pw_fwi* p, int nb_, int sg, float** Ap, float** Bp)
 {
     const Acq& a = p->acq;
     if (int rc = multi_fields(p, true)) return rc;
-    if (!p->adj_sa) { p->adj_sa = p->A2; p->adj_sb = p->B2; }
     float *A = *Ap, *B = *Bp, *Sa = (float*)p->adj_sa, *Sb = (float*)p->adj_sb;
     const long long fld = (long long)p->nslot * p->fs;
     const int a0 = sg * p->K, b0 = std::min(a0 + p->K, a.nt);
@@ -3174,7 +3178,6 @@ int adjoint_segment(pw_fwi* p, int nb_, int sg, int mode, T** Ap, T** Bp, T* gra
     if constexpr (sizeof(T) == 4) {
         if (mode == 0 && I == 1 && multi_ok(p)) {
             if (int rc = multi_fields(p, true)) return rc;
-            if (!p->adj_sa) { p->adj_sa = p->A2; p->adj_sb = p->B2; }
             float* Sa = (float*)p->adj_sa;
             float* Sb = (float*)p->adj_sb;
             const long long ss = (long long)p->nslot * p->nzx;
