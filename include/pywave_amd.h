@@ -202,6 +202,11 @@ int pw_fwi_widths(pw_fwi *p, int *w);
  * faster), 1 (one kernel per time step, the plain method) or -2 (two steps per launch whatever the
  * timing; acoustic point-source plans) */
 int pw_fwi_set_steps_per_launch(pw_fwi *p, int n);
+/* time steps per launch of the plan's sweeps as it is set up now: s[0] forward, s[1] reference
+ * adjoint, s[2] exact adjoint.  Four-step launches follow from the plan's size and settings, two from
+ * the timing sweep (1 before it).  A plan on four-step launches uses the widths above only where it
+ * recomputes a segment of a checkpointed run.  No counterpart in the reference. */
+int pw_fwi_launch_steps(pw_fwi *p, int *s);
 /* force the step kernels' tile widths instead of timing them: w[0] forward, w[1] visco forward,
  * w[2] exact adjoint, w[3] reference adjoint, w[4] visco reference adjoint, each 4, 8 or 16 (one
  * step per launch; forward steps that store their term take w[0]); NULL returns to the timing sweep.  Identical results at every width except the

@@ -4049,6 +4049,16 @@ int pw_fwi_widths(pw_fwi* p, int* w)
     return PW_OK;
 }
 
+int pw_fwi_launch_steps(pw_fwi* p, int* s)
+{
+    if (!p || !s) return PW_ERR_ARG;
+    const bool multi = multi_ok(p);
+    s[0] = multi ? kMulti : fused2(p) ? 2 : 1;
+    s[1] = multi && p->acq.interval == 1 ? kMulti : 1;
+    s[2] = multi ? kMulti : fused2_adj(p) ? 2 : 1;
+    return PW_OK;
+}
+
 int pw_fwi_tuning_log(pw_fwi* p, float* out, int cap)
 {
     if (!p) return PW_ERR_ARG;

@@ -128,7 +128,8 @@ class FwiProblem:
     def widths(self):
         """Tile widths of the step kernels picked by the plan's timing sweep (its first sweep runs
         it): forward, visco forward, exact adjoint, reference adjoint, visco reference adjoint, and
-        the forward steps that store their term for the exact adjoint."""
+        the forward steps that store their term for the exact adjoint.  Plans on four-step launches
+        (launch_steps) run these kernels only to recompute segments of a checkpointed run."""
         w = np.zeros(9, np.int32)
         N.check(self._L.pw_fwi_widths(self._p, N.ptr(w)), self._ctx, "widths")
         keys = ["forward", "visco_forward", "exact_adjoint", "reference_adjoint", "visco_reference_adjoint"]
@@ -160,6 +161,13 @@ class FwiProblem:
         the plan's timing sweep finds them faster), 1 (one kernel per time step, the plain method) or
         -2 (two steps per launch whatever the timing, on acoustic point-source plans)."""
         N.check(self._L.pw_fwi_set_steps_per_launch(self._p, int(n)), self._ctx, "set_steps_per_launch")
+
+    def launch_steps(self):
+        """Time steps per launch of the plan's forward, reference-adjoint and exact-adjoint sweeps as it
+        is set up now (two-step launches follow from the timing sweep, which the first call runs)."""
+        s = np.zeros(3, np.int32)
+        N.check(self._L.pw_fwi_launch_steps(self._p, N.ptr(s)), self._ctx, "launch_steps")
+        return dict(zip(["forward", "reference_adjoint", "exact_adjoint"], (int(x) for x in s)))
 
     def timing(self):
         f, b = ctypes.c_double(), ctypes.c_double()

@@ -378,6 +378,7 @@ def test_four_step_launches_equal_single_steps(nz, nx, ns, nb, nt, ckpt, acqui):
             p = FwiProblem(par, wav, data=obs, batch=batch, checkpoint=ckpt)
             p.set_steps_per_launch(steps)
             out.append((p.forward(vel),) + p.gradient(vel, "reference"))
+            assert set(p.launch_steps().values()) == {4 if steps == 2 else 1}
             p.close()
         (d4, g4, f4, s4), (d1, g1, f1, s1) = out
         assert np.array_equal(d4, d1) and d1.any()
@@ -389,5 +390,39 @@ def test_four_step_launches_equal_single_steps(nz, nx, ns, nb, nt, ckpt, acqui):
         p = FwiProblem(par, wav, data=obs, checkpoint=ckpt)
         p.set_steps_per_launch(steps)
         e.append(p.gradient(vel, "exact"))
+        assert set(p.launch_steps().values()) == {4 if steps == 2 else 1}
         p.close()
     assert e[0][1] == e[1][1] and rel_l2(e[0][0], e[1][0]) <= nt * 2e-7
+
+
+def test_which_plans_take_four_step_launches():
+    # at most 512 tiles of 32 x 16 cells over the shots of a launch; snapshots every other step leave the
+    # reference adjoint on single steps, and its gradient equals the single-step launches' bit for bit
+    par = dict(nz=130, nx=131, dz=0.01, dx=0.012, oz=0, ox=0, ns=5, ds=0.036, os=0.06, sz=5, nt=16, dt=0.001, ot=0,
+               nb=33, coef=0.005, acqui_type=1, interval=2, f0=10, inv=0, niter=2)
+    rng = np.random.default_rng(8)
+    vel = (1.5 + 1.5 * rng.random((130, 131))).astype(np.float32)
+    wav = (1e6 * rng.standard_normal(16)).astype(np.float32)
+    obs = rng.standard_normal((16, 131, 5)).astype(np.float32)
+    out = []
+    for steps in (2, 1):
+        p = FwiProblem(par, wav, data=obs)
+        p.set_steps_per_launch(steps)
+        n = 4 if steps == 2 else 1
+        assert p.launch_steps() == dict(forward=n, reference_adjoint=1, exact_adjoint=n)  # 455 tiles
+        out.append(p.gradient(vel, "reference"))
+        p.close()
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1:] == out[1][1:]
+    for change in (dict(ns=6), dict(precision="f64")):  # 546 tiles; the kernels' other precision
+        kw = {k: v for k, v in change.items() if k == "precision"}
+        p = FwiProblem(dict(par, **{k: v for k, v in change.items() if k == "ns"}), wav, **kw)
+        assert 4 not in p.launch_steps().values()
+        p.close()
+    p = FwiProblem(par, wav)
+    p.set_widths(8)
+    assert 4 not in p.launch_steps().values()
+    p.set_widths(timed=True)
+    assert p.launch_steps()["forward"] == 4
+    p.set_visco(np.full((130, 131), 50.0))
+    assert 4 not in p.launch_steps().values()
+    p.close()
