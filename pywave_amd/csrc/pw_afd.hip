@@ -1368,16 +1368,20 @@ int max_chunk_planes(const Geo& g)
 // blocks keep more of a plane's latencies in flight), of 16 rows beyond it (fewer halo re-reads):
 // with default_chunk, us per step on 91^3, 141^3, 201^3, 261^3 and 321^3 updated cells 6.7, 12.8,
 // 25.3, 42.7 and 122 with 8 rows, 100 at 321^3 with 16; one round of resident blocks of 16 rows,
-// 8 waves, the former choice, 11.5, 15.5, 31.4, 52 and 141.
+// 8 waves, the former choice, 11.5, 15.5, 31.4, 52 and 141.  Beyond those grids, with 16 rows against
+// the former choice: 335 against 456 on 460^3, 899 against 1380 on 660^3, 2051 against 3008 on 840^3; on
+// flat ones (z x y) 395 against 456 on 1060 x 1060 x 100, 269 against 290 on 1060 x 1060 x 65, 798
+// against 1317 on 65 x 1560 x 1560, 482 against 721 on 1560 x 65 x 1560.
 int default_variant(const pw_afd* p)
 {
     if (p->chunk_ok) return 3.0 * 4.0 * (double)p->field_elems <= kCacheFitBytes ? 15 : 17;
     return p->lean_ok ? kLeanOnlyDefault : kGeneralDefault;
 }
 
-// y planes per block with default_variant's pipelined kernels: about 35 chunks, of 3 to 8 planes.  The
-// best of 2 to 24 planes was 3, 3, 4, 5, 6, 6 and 8 on 91^3, 110^3, 141^3, 170^3, 201^3, 230^3 and
-// 261^3 updated cells, 5 on 141 x 100 x 160, 8 on 321^3.
+// y planes per block with default_variant's pipelined kernels: about 35 chunks, of 3 to 8 planes.  It
+// gives 3, 3, 4, 5, 6, 7, 7 and 8 on 91^3, 110^3, 141^3, 170^3, 201^3, 230^3, 261^3 and 321^3 updated
+// cells, where the best of 2 to 24 planes measured was 3, 3, 4, 5, 6, 6, 8 and 8; 5 on 141 x 100 x 160
+// (y last) is the best there too.
 int default_chunk(const Geo& g) { return std::min(8, std::max(3, (g.ny + 17) / 35)); }
 
 // whether 3D variant vi can run on this plan's grid
@@ -1514,6 +1518,10 @@ struct Shape2 {
     int k, owned_z, owned_x;
 };
 constexpr Shape2 kShapes2[] = {{8, 32, 8}, {8, 32, 16}, {8, 32, 32}, {4, 48, 16}};
+// On either side of the line, us per step of the four shapes (tiles): 240^2 1.23 (240), 1.25, 1.43,
+// 1.55; 300^2 1.43 (380), 1.30 (190), 1.44, 1.56; 263 x 457 1.82 (522), 1.37 (261), 1.50, 1.57; 360 x 460
+// 2.00, 1.51 (348), 1.51 (180), 1.53; 500^2 2.93, 1.61 (512), 1.47 (256), 2.03; 520^2 2.99, 2.15, 2.31
+// (289), 2.09.
 constexpr int kTilesAtOnce = 280;  // 256 CUs, and a few tiles that share one
 
 int shape2_of(const Geo& g)

@@ -2301,7 +2301,7 @@ struct pw_fwi {
     int w_fwdt = kDefaultWidth;  // forward steps that store their term for the exact adjoint
     int w_fwd2 = 0;       // two-step forward tiles' width (0: single steps are faster or not allowed)
     int w_adj2 = 0;       // two-step exact adjoint's width (0: single steps)
-    int max_fused = 2;    // forward steps one launch may advance (1: one kernel per time step)
+    int max_fused = 2;    // 1: one kernel per time step; 2: two, or four where multi_ok holds
     bool force_fused = false;  // two steps per launch whether or not they time faster
     std::vector<float> tune_log;  // (kernel, width, ms per launch) of the last timing sweep
     bool widths_tuned = false;
@@ -2617,6 +2617,9 @@ bool fused2_adj(const pw_fwi* p) { return p->max_fused >= 2 && p->w_adj2 > 0 && 
 //   101 x 203, 3 (441)    3.85 / 4.82   5.22 / 6.20
 //   200 x 300, 2 (540)    5.10 / 5.35   5.20 / 6.12
 //   400 x 800, 1 (986)    6.55 / 9.32   5.83 / 7.00
+// With a sponge of 30: 101 x 203, 5 (510) 3.97 / 5.13 against 5.56 / 6.30 and the exact adjoint 3.63
+// against 6.41; 160 x 240, 4 (532) 5.05 / 5.70 against 5.86 / 6.44; 200 x 300, 3 (621) 5.27 / 6.76 against
+// 5.97 / 6.40.
 // (Two steps per launch in tiles of 48 x 32 reached 4.5 forward on 200 x 300, 2 shots, and lost
 // everywhere else.)
 bool multi_ok(const pw_fwi* p)

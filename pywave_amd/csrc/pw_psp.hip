@@ -23,13 +23,13 @@
 // and inverse transform, the leapfrog update of its cells, and the new field's forward transform,
 // so the spectral Laplacian and the new field are never re-read from memory.
 //
-// Measured on the 144^3 grid (141^3 updated, 73 bins along z), us per launch: x forward 8.8, y 16.4,
-// x inverse 12.0, z columns 24, 59 per step, against 131 in six launches with one pass per level,
-// all transforms through LDS and the bins at a stride of 73.  Half of that came from the stride:
+// Measured on the 144^3 grid (141^3 updated, 73 bins along z), us per launch under the tracer: x forward
+// 8.8, y 16.0, x inverse 12.3, z columns 26.3; a step of a run 61, against 131 in six launches with one
+// pass per level, all transforms through LDS and the bins at a stride of 73.  Half of that came from the stride:
 // with 73 bins every 128 B segment of a 16-line load straddles two cache lines (a plain copy in
 // this order 12.8 us per 25 MB, 5.4 us at a stride of 80).  Bound now: about 72 MB a step through
 // the z kernel and 27 MB through each line pass, at 3 to 4 TB/s with the launch's ramp; on small 2D
-// grids (18 us against 38 for 192 x 240) the chain of latencies of a single wave per line.
+// grids (17 us against 37 for 192 x 240) the chain of latencies of a line's passes.
 #include <algorithm>
 #include <cmath>
 #include <string>
@@ -616,7 +616,7 @@ void launch_z(const PsLap* P, const PsStep& a, int inv, int fwd, hipStream_t s, 
 
 // Lines per block: 16 (128 B segments) where at least two blocks per CU remain and the buffers
 // leave room for several blocks per CU, else fewer.  Measured, 16 against 8 and 4 lines along x and
-// y and along z: 144^3 (141^3 updated) 59, 76 and 100 us a step, 120^3 40, 53 and 67 us; one line
+// y and along z: 144^3 (141^3 updated) 61, 76 and 100 us a step, 120^3 40, 53 and 67 us; one line
 // (64 threads) against four on the 2D 192 x 240 grid 17.9 against 20.5 (x) and 22.7 us (z).
 int lines_per_block(long long lines, int others, size_t (*lds)(int, int), int n)
 {
