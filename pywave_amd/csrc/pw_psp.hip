@@ -311,6 +311,8 @@ constexpr int z_stride(int lpb) { return lpb > 1 ? lpb + 1 : 1; }
 
 __device__ __forceinline__ float damp_axis(float v, float2 a) { return (v * a.x) * a.y; }
 
+constexpr int kFew = 4, kNear = 256;  // sources a block looks at without listing them; sources it can list
+
 // One time step of LPB neighbouring z columns (x0 .. x0+LPB-1 of plane y): split and half-length
 // inverse transform of their bins, centering sign and 1/(n1 n2 n3) -> the spectral Laplacian of
 // C_n; psm2d/psm's update of the columns' cells (pywave/src/wave_psp.c:518-581, :193-256):
@@ -319,7 +321,8 @@ __device__ __forceinline__ float damp_axis(float v, float2 a) { return (v * a.x)
 // forward transform of 'cur' (the first step's), fwd = 0 stops after the update (the last step).
 // Lanes run along z for global accesses and over columns in the passes; LDS elements are
 // LPB + 1 apart so both orders spread over the banks.
-template <bool D3, int LPB, int NT>
+// MANY: more than kFew sources.
+template <bool D3, int LPB, int NT, bool MANY>
 __global__ __launch_bounds__(NT, LPB >= 8 ? 6 : 1) void k_ps_z(FftDev arg, PsGeo g, PsStep a, cf* __restrict__ tmp,
                                              const cf* __restrict__ sup, int inv, int fwd)
 {
@@ -349,9 +352,29 @@ __global__ __launch_bounds__(NT, LPB >= 8 ? 6 : 1) void k_ps_z(FftDev arg, PsGeo
     const float* __restrict__ vv = a.vv + f0;
     cf* __restrict__ X = tmp + (long long)y * g.ldp + x0 * g.ldk;
     const unsigned col = (unsigned)c * g.ldz, xc = (unsigned)c * g.ldk;
-    bool hit = false;  // a source's stencil reaches the block's columns
-    for (int s = 0; s < a.ns; ++s)
-        hit |= abs(y - a.src[3 * s + 2]) <= 1 && a.src[3 * s + 1] >= x0 - 1 && a.src[3 * s + 1] <= x0 + LPB;
+    // The sources whose stencil reaches the block's columns, in source order: all of a few if one does;
+    // of many, those that do, found by the first wave 64 at a time.  (With every cell of such a block
+    // looking at all of 1000 sources a 2D step on 263 x 457 cells took 344 us, 31 with the list, 21 with
+    // one source; the list, at hand for one source too, cost a 3D step 3 %.)
+    __shared__ int near[MANY ? kNear + 1 : 1];  // their number, and which
+    auto reach = [&](int s) {
+        return abs(y - a.src[3 * s + 2]) <= 1 && a.src[3 * s + 1] >= x0 - 1 && a.src[3 * s + 1] <= x0 + LPB;
+    };
+    bool hit = false;
+    if constexpr (!MANY) {
+        for (int s = 0; s < a.ns; ++s) hit |= reach(s);
+    } else if (tid < 64) {
+        int n = 0;
+        for (int s0 = 0; s0 < a.ns; s0 += 64) {
+            const int s = s0 + tid;
+            const bool on = s < a.ns && reach(s);
+            const unsigned long long m = __ballot(on);
+            const int k = n + __popcll(m & ((1ull << tid) - 1));
+            if (on && k < kNear) near[1 + k] = s;
+            n += __popcll(m);
+        }
+        if (tid == 0) near[0] = n;
+    }
     const bool neg = g.n3 > 1 ? ((y & 1) != (x & 1)) : (x & 1);
     const float2 one = make_float2(1.f, 1.f);
     const float2 fxx = upd ? a.fx[x] : one, fyy = D3 && upd ? a.fy[y] : one;
@@ -418,13 +441,17 @@ __global__ __launch_bounds__(NT, LPB >= 8 ? 6 : 1) void k_ps_z(FftDev arg, PsGeo
     const bool model = x >= a.nb && x < a.nb + a.nx1 && y >= nby && y < nby + a.ny1;
     const long long r = (long long)(y - nby) * a.nx1 + (x - a.nb);
     const float w = neg ? -g.wwt : g.wwt;
+    // (the list was published by the barriers of the inverse transform)
+    const int listed = MANY && inv ? __builtin_amdgcn_readfirstlane(near[0]) : 0;
+    const int nsrc = !MANY ? (hit ? a.ns : 0) : listed <= kNear ? listed : a.ns;
     auto cell = [&](int z, float u, float p, float vc) {
         const float2 fzz = fz[z];
         p = damp_axis(damp_axis(p, fzz), fxx);
         if (D3) p = damp_axis(p, fyy);
         float v = u + (u - p);
         v = v + (w * Bf[at(z)]) * vc;
-        for (int s = 0; hit && s < a.ns; ++s) {
+        for (int i = 0; i < nsrc; ++i) {
+            const int s = MANY && listed <= kNear ? __builtin_amdgcn_readfirstlane(near[1 + i]) : i;
             const int dz = abs(z - a.src[3 * s]), dx = abs(x - a.src[3 * s + 1]), dy = abs(y - a.src[3 * s + 2]);
             if (dz <= 1 && dx <= 1 && dy <= 1)
                 v = v + (vc * a.wav[(size_t)s * a.nt + a.it]) / (float)(dz + dx + dy + 1);
@@ -602,16 +629,21 @@ void launch_z(const PsLap* P, const PsStep& a, int inv, int fwd, hipStream_t s, 
     const int lpb = P->lz;
     const dim3 grid((unsigned)((g.n2 + lpb - 1) / lpb), (unsigned)g.n3);
     const size_t lds = z_lds(g.h, lpb);
-    if (lpb == 16)
-        hipExtLaunchKernelGGL((k_ps_z<D3, 16, 256>), grid, dim3(256), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
-    else if (lpb == 8)
-        hipExtLaunchKernelGGL((k_ps_z<D3, 8, 128>), grid, dim3(128), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
-    else if (lpb == 4)
-        hipExtLaunchKernelGGL((k_ps_z<D3, 4, 64>), grid, dim3(64), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
-    else if (g.h > kLongColumn)
-        hipExtLaunchKernelGGL((k_ps_z<D3, 1, 512>), grid, dim3(512), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
-    else
-        hipExtLaunchKernelGGL((k_ps_z<D3, 1, 256>), grid, dim3(256), lds, s, e0, e1, 0, P->z, g, a, P->tmp, P->sup, inv, fwd);
+#define PW_PSZ(LPB, NT)                                                                                       \
+    do {                                                                                                      \
+        if (a.ns > kFew)                                                                                      \
+            hipExtLaunchKernelGGL((k_ps_z<D3, LPB, NT, true>), grid, dim3(NT), lds, s, e0, e1, 0, P->z, g, a, \
+                                  P->tmp, P->sup, inv, fwd);                                                  \
+        else                                                                                                  \
+            hipExtLaunchKernelGGL((k_ps_z<D3, LPB, NT, false>), grid, dim3(NT), lds, s, e0, e1, 0, P->z, g,   \
+                                  a, P->tmp, P->sup, inv, fwd);                                               \
+    } while (0)
+    if (lpb == 16) PW_PSZ(16, 256);
+    else if (lpb == 8) PW_PSZ(8, 128);
+    else if (lpb == 4) PW_PSZ(4, 64);
+    else if (g.h > kLongColumn) PW_PSZ(1, 512);
+    else PW_PSZ(1, 256);
+#undef PW_PSZ
 }
 
 // Lines per block: 16 (128 B segments) where at least two blocks per CU remain and the buffers

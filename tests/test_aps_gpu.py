@@ -162,3 +162,30 @@ def test_aps_long_lines_vs_oracle(shape):
     assert np.array_equal(out[:n].reshape((nt,) + shape[1:], order="F"), d.T)
     w = out[n:].reshape(shape + (-1,), order="F")
     assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
+
+
+@pytest.mark.parametrize("shape,ns", [((30, 25), 4), ((30, 25), 5), ((30, 25), 130), ((40, 6), 700), ((84, 83, 85), 300)])
+def test_aps_many_sources_vs_oracle(shape, ns):
+    # source counts on either side of those that a block of columns lists (more than 4 in all, up to 256
+    # that reach it: 700 over six columns exceed that), several on one cell: added in source order as the
+    # oracle does, so equal
+    rng = np.random.default_rng(ns)
+    nt, dt, nbt, d2, d3 = 5, 0.0005, 5, (9.0, 10.0), (12.0, 10.0, 11.0)
+    vel = (1700 + 900 * rng.random(shape)).astype(np.float32)
+    wav = rng.standard_normal((ns, nt)).astype(np.float32)
+    s = [rng.integers(0, n, ns) for n in shape[1:] + shape[:1]]
+    for c in s:
+        c[-2:] = c[0]
+    l = [list(c) for c in s]
+    if len(shape) == 2:
+        d, snaps, _ = O.afd2d(vel, nt, dt, d2[1], d2[0], nbt, 0.03, l[0], l[1], wav, jsnap=4, ps=True)
+    else:
+        d, snaps, _ = O.afd3d(vel, nt, dt, d3[1], d3[2], d3[0], nbt, 0.03, l[0], l[1], l[2], wav, jsnap=4, ps=True)
+    p = AfdPlan(vel, d2 if len(shape) == 2 else d3, nt, dt, nbt, 0.03, 4, spectral=True)
+    p.set_sources(np.concatenate(s + [np.full(ns, 25), np.full(ns, 0.002), np.ones(ns)]).astype(np.float32), ns, wavelet=wav)
+    p.run()
+    out = p.output()
+    n = nt * int(np.prod(shape[1:]))
+    assert np.array_equal(out[:n].reshape((nt,) + shape[1:], order="F"), d.T)
+    w = out[n:].reshape(shape + (-1,), order="F")
+    assert all(np.array_equal(w[..., k], snaps[k].T) for k in range(w.shape[-1]))
