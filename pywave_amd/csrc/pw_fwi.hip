@@ -2227,7 +2227,11 @@ void residual_weights(const Acq& a, std::vector<float>& w /* [ir][it] */)
     float sw[10];
     for (int it = 0; it < 10; ++it) sw[it] = sinf(0.5 * PI_D * (it + 1) / 11.);
     w.assign((size_t)nt * nr, 0.f);
-    auto W = [&](int ir, int it) -> float& { return w[(size_t)ir * nt + it]; };
+    float off = 0.f;  // tapers of fewer than 10 receivers or samples run past the array
+    auto W = [&](int ir, int it) -> float& {
+        const long long i = (long long)ir * nt + it;
+        return i >= 0 && i < (long long)nt * nr ? w[(size_t)i] : off;
+    };
     for (int ir = woffn1; ir <= woffn2; ++ir)
         for (int it = wtn1; it <= wtn2; ++it) W(ir, it) = 1.;
     for (int ir = 0; ir < 10; ++ir)

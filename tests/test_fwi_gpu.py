@@ -426,3 +426,22 @@ def test_which_plans_take_four_step_launches():
     p.set_visco(np.full((130, 131), 50.0))
     assert 4 not in p.launch_steps().values()
     p.close()
+
+
+@pytest.mark.parametrize("nx,nt", [(7, 40), (40, 8), (6, 5)])
+def test_gradients_of_fewer_than_ten_receivers_or_samples(nx, nt):
+    # the residual weights' 10-sample tapers reach past such data: a plan's arrays stay intact and its
+    # four-step and single-step launches agree
+    rng = np.random.default_rng(nx + nt)
+    par = dict(nz=20, nx=nx, dz=0.01, dx=0.01, oz=0, ox=0, ns=1, ds=0.01, os=0.02, sz=5, nt=nt, dt=0.001, ot=0, nb=12,
+               coef=0.005, acqui_type=1, interval=1, f0=10, inv=0, niter=1)
+    vel = (1.5 + rng.random((20, nx))).astype(np.float32)
+    wav = (1e6 * rng.standard_normal(nt)).astype(np.float32)
+    obs = rng.standard_normal((nt, nx, 1)).astype(np.float32)
+    out = []
+    for steps in (2, 1):
+        p = FwiProblem(par, wav, data=obs)
+        p.set_steps_per_launch(steps)
+        out.append((p.forward(vel), p.gradient(vel, "reference")[0]))
+        p.close()
+    assert np.isfinite(out[0][1]).all() and np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
