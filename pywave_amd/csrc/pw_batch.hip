@@ -661,7 +661,10 @@ int pw_batch2d_traces(pw_batch* p, int i, float* out, long long len)
     if (len != (long long)s.nt * s.nx1) PW_FAIL(p->ctx, PW_ERR_ARG, "batch traces: length mismatch");
     hipStream_t st = p->ctx->s();
     if (int rc = pw::check_finite(p->ctx, p->d_rec + s.rec_off, (size_t)len, 4, "batch2d: receiver traces")) return rc;
-    if (!p->d_out) {  // one shot's transposed traces, sized for the largest
+    // the host's loop is the faster way for few samples (60 x 100: 38 us a call against 48, 60 x 400: 45
+    // against 51, 200 x 400: 70 against 61)
+    constexpr long long kHostSamples = 32 * 1024;
+    if (!p->d_out && len > kHostSamples) {  // one shot's transposed traces, sized for the largest
         long long most = 0;
         for (const Shot& q : p->shots) most = std::max(most, (long long)q.nt * q.nx1);
         const pw::OnDevice dev(p->ctx);
@@ -670,7 +673,7 @@ int pw_batch2d_traces(pw_batch* p, int i, float* out, long long len)
             p->d_out = nullptr;
         }
     }
-    if (!p->d_out) {  // no room on the device for the run's traces in the callers' order
+    if (!p->d_out || len <= kHostSamples) {  // or no room on the device for them in the callers' order
         std::vector<float> t((size_t)len);
         PW_HIP(p->ctx, hipMemcpyAsync(t.data(), p->d_rec + s.rec_off, len * 4, hipMemcpyDeviceToHost, st));
         PW_HIP(p->ctx, hipStreamSynchronize(st));
