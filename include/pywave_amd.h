@@ -274,7 +274,8 @@ int pw_lstri_steps_per_launch(pw_lstri *p, int n);
 /* single-step tile width (x columns per 64-cell tile): 1, 2, 4, 8, 16, or 0 for the plan's timed
  * choice; identical results either way.  No counterpart in the reference. */
 int pw_lstri_set_tile_width(pw_lstri *p, int w);
-/* columns per wave of the four-step launches: 4 (tiles of 16), 8 (of 32), or 0 for the timed choice (identical
+/* columns per wave of the four-step launches: 4 (tiles of 16), 8 (of 32), or 0 for the timed choice, with
+ * which the adjoint of grids of up to 256 tiles of 56 x 4 cells runs in LDS tiles instead (identical
  * results).  No counterpart in the reference. */
 int pw_lstri_set_four_step_columns(pw_lstri *p, int c);
 /* the last sweep's launch choice: w[0] single-step tile width, w[1] steps per launch, w[2] the

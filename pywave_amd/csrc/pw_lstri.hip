@@ -626,6 +626,112 @@ __global__ __launch_bounds__(64 * trn_waves(S)) void k_trn(TriGeo g, TriArgsN<NS
     }
 }
 
+// ---------------------------------------------------------------- four adjoint steps of small grids
+// The adjoint's four steps in a tile kept wholly in LDS: a block owns 56 x 4 cells and forms step k on
+// the tile grown by 4*(4-k), so on grids whose tiles have a CU each it computes fewer cells than a strip
+// tile, which works on whole 64-lane columns (both are bound there by one tile's VALU work and LDS
+// latency).  LA/PA hold the even levels and their products with v^2dt^2, LB/PB the odd ones; a step
+// overwrites, cell by cell, the level it reads pointwise.  Same expressions per cell as single steps.
+// Measured, us per launch, against strips of 4 columns: 31 x 33 cells 6.8 and 7.7, 100 x 120 7.2 and
+// 8.0; of the modelling steps, which stage each step's source plane too, strips are the faster form
+// everywhere (7.6 and 8.3 against 8.0 and 8.7).
+constexpr int kTileZ = 56, kTileX = 4;  // owned cells
+
+__global__ __launch_bounds__(1024) void k_tra_tile(TriGeo g, TriArgsN<NSN> a, int ntz)
+{
+    constexpr int NS = NSN, TN = 1024, OZ = kTileZ, OX = kTileX, G = 4 * NS;
+    constexpr int ZA = OZ + 2 * G, XA = OX + 2 * G;              // staged region R_0
+    constexpr int ZB = OZ + 2 * (G - 4), XB = OX + 2 * (G - 4);  // R_1
+    __shared__ float LA[XA][ZA + 1], PA[XA][ZA + 1], VV[XA][ZA + 1];
+    __shared__ float LB[XB][ZB + 1], PB[XB][ZB + 1];
+    __shared__ float fz[ZA], fx[XA];  // decay factors (one of a pair is 1)
+    __shared__ float rd[NS][XB];      // each step's injected row
+    const int slot = blockIdx.y;
+    const int tz = blockIdx.x % ntz, tx = blockIdx.x / ntz;
+    const int zo = tz * OZ, xo = tx * OX;
+    const long long so = slot * g.fs;
+    auto ing = [&](int z, int x) { return z >= 0 && z < g.pz && x >= 0 && x < g.px; };
+    auto mx = [&](int x) { return x >= g.nb && x < g.nb + g.nx; };
+    // every global operand into registers first, so the launch waits on memory once
+    constexpr int N0 = (ZA * XA + TN - 1) / TN, N1 = (ZB * XB + TN - 1) / TN;
+    float r0[N0], rv[N0], r1[N1];
+#pragma unroll
+    for (int j = 0; j < N0; ++j) {
+        const int e = threadIdx.x + j * TN, z = zo - G + e % ZA, x = xo - G + e / ZA;
+        const bool in = e < ZA * XA && ing(z, x);
+        const long long k = (long long)x * g.ldz + z;
+        r0[j] = in ? a.X[so + k] : 0.f;
+        rv[j] = in ? a.v2[k] : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < N1; ++j) {
+        const int e = threadIdx.x + j * TN, z = zo - G + 4 + e % ZB, x = xo - G + 4 + e / ZB;
+        r1[j] = e < ZB * XB && ing(z, x) ? a.Y[so + (long long)x * g.ldz + z] : 0.f;
+    }
+    for (int e = threadIdx.x; e < NS * XB; e += TN) {
+        const int x = xo - G + 4 + e % XB;
+        rd[e / XB][e % XB] = mx(x) ? a.row[e / XB][slot * a.rss + (x - g.nb)] : 0.f;
+    }
+    for (int t = threadIdx.x; t < ZA + XA; t += TN) {
+        const int z = zo - G + t, x = xo - G + t - ZA;
+        if (t < ZA) fz[t] = z >= 0 && z < g.pz ? a.sfz[2 * z] * a.sfz[2 * z + 1] : 1.f;
+        else fx[t - ZA] = x >= 0 && x < g.px ? a.sfx[2 * x] * a.sfx[2 * x + 1] : 1.f;
+    }
+#pragma unroll
+    for (int j = 0; j < N0; ++j) {
+        const int e = threadIdx.x + j * TN;
+        if (e < ZA * XA) {
+            LA[e / ZA][e % ZA] = r0[j];
+            VV[e / ZA][e % ZA] = rv[j];
+            PA[e / ZA][e % ZA] = r0[j] * rv[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < N1; ++j) {
+        const int e = threadIdx.x + j * TN;
+        if (e < ZB * XB) LB[e / ZB][e % ZB] = r1[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 1; k <= NS; ++k) {
+        const int zr = OZ + 8 * (NS - k), xr = OX + 8 * (NS - k);
+        const int da = 4 * k, db = 4 * (k - 1);  // the region's offsets in R_0 and R_1 coordinates
+        const bool odd = k & 1;                  // level k goes to LB (odd) or LA (even)
+        for (int e = threadIdx.x; e < zr * xr; e += TN) {
+            const int zz = e % zr, xx = e / zr;
+            const int z = zo - 4 * (NS - k) + zz, x = xo - 4 * (NS - k) + xx;
+            const int za = zz + da, xa = xx + da, zb = zz + db, xb = xx + db;
+            float v = 0.f, pv = 0.f;
+            if (ing(z, x)) {
+                const bool own = z >= zo && z < zo + OZ && x >= xo && x < xo + OX;
+                const float vv = VV[xa][za], f = fz[za], h = fx[xa];
+                const float u1 = odd ? LA[xa][za] : LB[xb][zb], prev = odd ? LB[xb][zb] : LA[xa][za];
+                const float c = odd ? PA[xa][za] : PB[xb][zb];
+                if (own && mx(x) && z >= g.nb && z < g.nb + g.nz)  // this step's image
+                    a.plane[k - 1][slot * a.pss + (long long)(x - g.nb) * g.nz + (z - g.nb)] = 0.f + c;
+                float u2 = 0.f;  // the 4-cell rim stays zero
+                if (z >= 4 && z < g.pz - 4 && x >= 4 && x < g.px - 4) {
+                    auto at = [&](int dx, int dz) { return odd ? PA[xa + dx][za + dz] : PB[xb + dx][zb + dz]; };
+                    const float lx = W4 * (at(4, 0) + at(-4, 0)) + W3 * (at(3, 0) + at(-3, 0)) +
+                                     W2 * (at(2, 0) + at(-2, 0)) + W1 * (at(1, 0) + at(-1, 0)) + W0 * c;
+                    const float lz = W4 * (at(0, 4) + at(0, -4)) + W3 * (at(0, 3) + at(0, -3)) +
+                                     W2 * (at(0, 2) + at(0, -2)) + W1 * (at(0, 1) + at(0, -1)) + W0 * c;
+                    u2 = (lx * g.sx + lz * g.sz) + 2.0f * u1 - h * (f * prev);
+                }
+                if (z == g.depth && mx(x)) u2 = u2 + rd[k - 1][xb];
+                v = h * (f * u2);
+                pv = v * vv;
+                if (k >= NS - 1 && own) (k == NS ? a.D : a.C)[so + (long long)x * g.ldz + z] = v;
+            }
+            if (k < NS) {  // over the level this cell read pointwise (no other cell reads it now)
+                (odd ? LB[xb][zb] : LA[xa][za]) = v;
+                (odd ? PB[xb][zb] : PA[xa][za]) = pv;
+            }
+        }
+        if (k < NS) __syncthreads();
+    }
+}
+
 // ---------------------------------------------------------------- small kernels
 __global__ void k_tri_pad_v2(TriGeo g, const float* __restrict__ vel, float dt2, float* __restrict__ v2)
 {
@@ -866,8 +972,18 @@ void launch_trn(pw_lstri* p, bool adj, int nslot, const TriArgsN<NSN>& a)
     else hipLaunchKernelGGL((k_trn<false, NSN, S>), grid, block, 0, p->ctx->s(), p->g, a, ntz);
 }
 
+// Tiles up to which k_tra_tile takes the adjoint's four steps (a CU each), unless a strip width was asked
+// for.  Per launch against 4-column strips: 180 tiles 7.2 against 8.2 us, 260 7.7 against 8.3, 288 9.6
+// against 8.3, 450 10.2 against 8.4.
+constexpr int kTileLimit = 256;
+
 void step4(pw_lstri* p, bool adj, int nslot, const TriArgsN<NSN>& a)
 {
+    const int ntz = (p->g.pz + kTileZ - 1) / kTileZ, ntx = (p->g.px + kTileX - 1) / kTileX;
+    if (adj && !p->oxn_forced && (long long)ntz * ntx * nslot <= kTileLimit) {
+        hipLaunchKernelGGL(k_tra_tile, dim3(ntz * ntx, nslot), dim3(1024), 0, p->ctx->s(), p->g, a, ntz);
+        return;
+    }
     if (p->oxn == 8) launch_trn<8>(p, adj, nslot, a);
     else launch_trn<4>(p, adj, nslot, a);
 }

@@ -218,3 +218,20 @@ def test_four_step_tiles_at_grid_edges_vs_single_steps(nz, nx, nb, cols):
     four.set_four_step_columns(cols)
     assert np.array_equal(one.model(src), four.model(src))
     assert np.array_equal(one.image(dat), four.image(dat))
+
+
+@pytest.mark.parametrize("nz,nx,nb,ns", [(7, 9, 12, 1), (38, 22, 9, 1), (39, 23, 9, 3), (100, 33, 4, 2), (100, 180, 20, 2)])
+def test_four_step_adjoint_of_small_grids_vs_single_steps(nz, nx, nb, ns):
+    # without a forced strip width the adjoint of grids of up to 256 tiles of 56 x 4 cells (9 to 54 here,
+    # padded grids equal to whole tiles and one cell beyond) runs in LDS tiles, the last grid (330) in
+    # strips: the same expressions per cell, so equal
+    rng = np.random.default_rng(nz + nx)
+    nt = 11
+    par = np.array([nz, nx, 0.01, 0.012, 0, 0, nt, 0.001, 0, 0, ns, 0.2, 0, 5, nb, 0.01, 10, 1, 1, 2], np.float32)
+    vel = (1.5 + 2 * rng.random((nz, nx))).astype(np.float32)
+    dat = rng.standard_normal((nt, nx, ns)).astype(np.float32)
+    one, four = LstriProblem(par, vel), LstriProblem(par, vel)
+    one.steps_per_launch(1)
+    four.steps_per_launch(4)
+    assert np.array_equal(one.image(dat), four.image(dat))
+    assert np.array_equal(one.invert(dat, 2), four.invert(dat, 2))
