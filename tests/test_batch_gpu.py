@@ -102,3 +102,21 @@ def test_every_tile_width_bit_exact_and_tuning_recorded():
     b2.run(False)
     assert b2.width() == (w, log)
     b2.close()
+
+
+@pytest.mark.parametrize("nx,nt", [(128, 256), (33, 993), (181, 182), (1, 33000)])
+def test_traces_transposed_on_host_and_device_vs_single_plans(nx, nt):
+    # 32768 samples (the most that the host transposes), one more, and sizes off the 32 x 32 tiles of the
+    # device's transpose: the single plans' traces, in the same order
+    rng = np.random.default_rng(nx)
+    vel = (1500 + 1500 * rng.random((12, nx))).astype(np.float32)
+    src = np.array([nx // 2, 5, 20, 0.002, 1], np.float32)
+    wav = rng.standard_normal((1, nt)).astype(np.float32)
+    b = pywave_amd.Afd2dBatch([dict(vel=vel, d=(10.0, 10.0), nt=nt, dt=0.001, src=src, ns=1, wavelet=wav)], nbt=5)
+    b.run()
+    p = pywave_amd.AfdPlan(vel, (10.0, 10.0), nt, 0.001, 5, 0.01, 0)
+    p.set_sources(src, 1, wavelet=wav)
+    p.run()
+    assert np.array_equal(b.traces(0), p.output().reshape(nt, nx, order="F"))
+    b.close()
+    p.close()
